@@ -2112,9 +2112,10 @@ __device__ __forceinline__ void gu_mfma(GuSmem<C>& sm, int W, int WR, int lo_h, 
   }
 }
 
-// MFMA down: rows [hb, hb + 16 NA) of a [H][KD] weight (nv of them real), all K steps, in
-// registers; mma() gives C[m][n] = row hb + 16 q + m against pick column n of an LDS mid tile,
-// for each of the NA 16-row blocks q
+// MFMA down: a unit of 16 NA rows of a [H][KD] weight, all K steps, in registers; mma() gives
+// C[m][n] = the unit's row 16 q + m against pick column n of an LDS mid tile, for each of the NA
+// 16-row blocks q. A routed unit's rows may belong to several experts (mfma_issue), each lane
+// addressing its own; the shared down's are rows [hb, hb + nv) of one weight (load)
 template <int WFMT, int KD, int NA_ = 1, bool SH = false, int KR = KD>
 struct DownTile {
   static constexpr int NA = NA_;  // 16-row A operands a unit
@@ -2140,57 +2141,75 @@ struct DownTile {
       (WFMT == kFp4 && KS >= 8) || BYTES >= 16384 ? 1 : (16384 / BYTES > 4 ? 4 : 16384 / BYTES);
   static_assert(NA == 1 || WFMT == kFp4, "FP8 units are one 16-row block");
   u32x4 a[NA][KS][NW];
-  // MXFP4: the E8M0 byte of the lane's row and block (load_scales<true>: the loaded dwords); MX
+  // MXFP4: the E8M0 byte of the lane's row and block (load_scales: the loaded dwords); MX
   // FP8: the lane's row block's codes of its two pieces' K blocks (low byte: 16 j .., next:
   // 64 + 16 j ..)
   uint32_t sa[NA][KS];
-  float s0[KS], s1[KS];  // FP8: block scales of the lane's first and last C row
-  int split;             // FP8: C elements v < split take s0, the rest s1
+  float s0[KS];  // FP8: the block scales of the lane's four C rows (rows 4 i .. 4 i + 3: one block)
 
   // The unit through LDS. issue() requests its 16 NA rows into a wave's slot by LDS-direct
-  // 16-byte loads, each load a contiguous KB of the weight (the operand layout's own loads read
+  // 16-byte loads, each load runs of whole rows of the weight (the operand layout's own loads read
   // 64-byte runs, which stream at about 5.1 against 6.6 TB/s: measured, loads alone). Chunk c
   // (16 bytes) of row r sits at slot position r * CPR + (c ^ (r % 16)), so that the 16 rows'
-  // reads of one chunk fall in distinct banks. Rows past nv are requested past the resource
-  // (zeros, no memory access). fetch() reads the slot into a[][] in the operand layout; the
-  // scales travel in registers (load_scales, take_scales).
+  // reads of one chunk fall in distinct banks. fetch() reads the slot into a[][] in the operand
+  // layout; the scales travel in registers (load_scales, take_scales).
   static constexpr int RB = F8 ? KD : KD / 2;  // bytes a row
   static constexpr int CPR = RB / 16;         // chunks a row
   static constexpr int SLOT = 16 * NA * RB;   // bytes a unit
-  // (row-major units through LDS: the swizzle needs CPR a power of two of 16 or more; the
-  // shuffled layout's blocks go in whole)
-  static constexpr bool kRowMajorSlot = CPR >= 16 && (CPR & (CPR - 1)) == 0 && SLOT % 1024 == 0;
-  // wr: a resource over the weight from row 0 (H x RB bytes a matrix); wrow: the unit's first
-  // row's byte offset in it
-  __device__ __forceinline__ static void issue(__amdgpu_buffer_rsrc_t wr, uint32_t wrow, int nv, uint8_t* slot,
-                                               int lane) {
+  // (row-major units through LDS: the swizzle needs CPR a power of two of 16 or more, at most a
+  // wave's 64 lanes; the shuffled layout's blocks go in whole)
+  static constexpr bool kRowMajorSlot = CPR >= 16 && CPR <= 64 && (CPR & (CPR - 1)) == 0 && SLOT % 1024 == 0;
+
+  // lane l's value of lanes' values v, where lanes 16 g + m hold row m's: row R's in the lanes
+  // [0, 64 / N), R + 1's in the next 64 / N and so on (N rows a 1 KB load; row_newbcast takes one
+  // lane of each 16-lane row to the whole row)
+  template <int R, int N>
+  __device__ __forceinline__ static uint32_t rows_to_runs(uint32_t v) {
+    static_assert(N == 1 || N == 2 || N == 4, "rows a load");
+    int o = __builtin_amdgcn_update_dpp(0, (int)v, 0x150 + R, 0xF, 0xF, true);
+    if constexpr (N == 2) o = __builtin_amdgcn_update_dpp(o, (int)v, 0x150 + R + 1, 0xC, 0xF, false);
+    if constexpr (N == 4) {
+      o = __builtin_amdgcn_update_dpp(o, (int)v, 0x150 + R + 1, 0x2, 0xF, false);
+      o = __builtin_amdgcn_update_dpp(o, (int)v, 0x150 + R + 2, 0x4, 0xF, false);
+      o = __builtin_amdgcn_update_dpp(o, (int)v, 0x150 + R + 3, 0x8, 0xF, false);
+    }
+    return (uint32_t)o;
+  }
+  // load I of block q of the row-major unit: rows I * 64 / CPR .. of the block
+  template <int I>
+  __device__ __forceinline__ static void issue_runs(__amdgpu_buffer_rsrc_t wr, uint32_t off, uint8_t* slot, int lane) {
+    constexpr int N = 64 / CPR, PER = 16 * RB / 1024;
+    if constexpr (I < PER) {
+      const int r = I * N + lane / CPR, c = (lane % CPR) ^ r;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(slot + I * 1024), 16,
+                                               rows_to_runs<I * N, N>(off) + c * 16, 0, 0, kAuxNt);
+      issue_runs<I + 1>(wr, off, slot, lane);
+    }
+  }
+  // wr: a resource over the whole weight; row[q]: the weight row of this lane's A row of block q
+  // (row l % 16; < 0: none, requested past the resource: zeros, no memory access)
+  __device__ __forceinline__ static void issue(__amdgpu_buffer_rsrc_t wr, const int (&row)[NA], uint8_t* slot, int lane) {
     if constexpr (SH) {
       // SGLang's layout: a row's 16-byte piece j of K step ks sits in its 16-row group's 1 KB
-      // block ks, at lane (row % 16) + 16 j (the unit's rows may straddle two groups). Slot
-      // block q KS + ks takes the unit's rows 16 q .. of K step ks in the operand's lane
-      // order, lane l's 16 bytes at 16 l
-      const int m = lane & 15, j = lane >> 4;
-      const uint32_t row0 = wrow / RB;
+      // block ks, at lane (row % 16) + 16 j. Slot block q KS + ks takes the rows of block q of K
+      // step ks in the operand's lane order, lane l's 16 bytes at 16 l
+      const int j = lane >> 4;
 #pragma unroll
       for (int q = 0; q < NA; ++q) {
-        const uint32_t row = row0 + q * 16 + m;
-        const uint32_t base = (row / 16) * 16 * RB + ((row % 16) + 16 * j) * 16;
+        const uint32_t base = ((uint32_t)row[q] / 16) * 16 * RB + (((uint32_t)row[q] % 16) + 16 * j) * 16;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
               wr, (__attribute__((address_space(3))) void*)(slot + (q * KS + ks) * 1024), 16,
-              q * 16 + m < nv && ks * 128 + 32 * j < KR ? base + ks * 1024 : kNoLoad, 0, 0, kAuxNt);
+              row[q] >= 0 && (ks * 128 + 128 <= KR || ks * 128 + 32 * j < KR) ? base + ks * 1024 : kNoLoad, 0, 0, kAuxNt);
       }
       return;
     }
     static_assert(SH || kRowMajorSlot, "slot layout");
+    if constexpr (kRowMajorSlot) {
 #pragma unroll
-    for (int i = 0; i < SLOT / 1024; ++i) {
-      const int pos = i * 64 + lane;
-      const int r = pos / CPR, c = (pos % CPR) ^ (r & 15);
-      const uint32_t off = r < nv ? wrow + (uint32_t)r * RB + c * 16 : kNoLoad;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(slot + i * 1024), 16,
-                                               off, 0, 0, kAuxNt);
+      for (int q = 0; q < NA; ++q)
+        issue_runs<0>(wr, row[q] >= 0 ? (uint32_t)row[q] * RB : kNoLoad, slot + q * 16 * RB, lane);
     }
   }
   __device__ __forceinline__ void fetch(const uint8_t* slot, int lane) {
@@ -2213,72 +2232,39 @@ struct DownTile {
           a[q][ks][w] = *(const u32x4*)(slot + ((q * 16 + m) * CPR + (c ^ m)) * 16);
         }
   }
-  // the unit's scales alone (as load() sets them). FP8: the 128 x 128 block scales of the
-  // lane's C rows; MXFP4: the lane's row's KD / 32 E8M0 bytes in 16-byte loads (byte j of
-  // dword ks is its block's), rows past nv unit scales. RAW (MXFP4): sa keeps the loaded
-  // dwords as they are and take_scales picks the lane's bytes out of them, so that nothing
-  // waits for the loads here: a wave's loads complete in order, so a wait for the scales
-  // would wait for the unit's weight rows requested just before them
-  template <bool RAW = false>
-  __device__ __forceinline__ void load_scales(const void* s, int hb, int nv, int lane) {
-    const int m = lane & 15, j = lane >> 4;
+  // The unit's scales, requested with its rows and left as they come until take_scales, so that
+  // nothing waits for the loads here: a wave's loads complete in order, so a wait for the scales
+  // would wait for the unit's weight rows requested just before them. sr: a resource over the
+  // whole scale tensor. FP8: the block scales of the lane's C rows, from word crow; MXFP4: the
+  // E8M0 bytes of this lane's A rows row[q] (byte j of dword ks is its block's; rows < 0: zeros)
+  __device__ __forceinline__ void load_scales(__amdgpu_buffer_rsrc_t sr, const int (&row)[NA], int cblk, int lane) {
+    const int j = lane >> 4;
     if constexpr (WFMT == kFp8) {
-      const int r0 = hb + min(4 * j, nv - 1), r3 = hb + min(4 * j + 3, nv - 1);
-      const float* sp = (const float*)s;
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        s0[ks] = sp[(r0 / 128) * (KD / 128) + ks];
-        s1[ks] = sp[(r3 / 128) * (KD / 128) + ks];
-      }
-      split = r0 / 128 == r3 / 128 ? 4 : 128 - (hb + 4 * j) % 128;
-    } else if constexpr (WFMT == kFp8Mx) {
-      // E8M0 [H / 32][KD / 32]: lane (m, j) supplies A row hb + m (a unit may straddle two
-      // 32-row blocks), its pieces of step ks in K blocks 4 ks + j / 2 and 4 ks + 2 + j / 2 (the
-      // second past the row in a half step)
-      const uint8_t* row = (const uint8_t*)s + (size_t)((hb + min(m, nv - 1)) / 32) * (KD / 32);
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int b0 = 4 * ks + (j >> 1), b1 = b0 + 2;
-        sa[0][ks] = row[b0] | (b1 < KD / 32 ? (uint32_t)row[b1] << 8 : 0u);
-      }
+      for (int ks = 0; ks < KS; ++ks)
+        s0[ks] = u2f(__builtin_amdgcn_raw_buffer_load_b32(sr, (uint32_t)(cblk + ks) * 4, 0, 0));
     } else if constexpr (SH) {
-      // shuffle_scale order (a [H][KD / 32] matrix of the expert): row h's bytes of K steps
-      // 2 c and 2 c + 1, column j of each, are bytes 2 (step % 2) + (h / 16) % 2 of the dword
-      // at 32-row block h / 32, chunk c (256 bytes), position 16 j + h % 16
-      const uint8_t* ss = (const uint8_t*)s;
+      // shuffle_scale order (a [rows][SC] matrix): row h's bytes of K steps 2 c and 2 c + 1,
+      // column j of each, are bytes 2 (step % 2) + (h / 16) % 2 of the dword at 32-row block
+      // h / 32, chunk c (256 bytes; with an odd KS the last holds one step), position 16 j + h % 16
 #pragma unroll
       for (int q = 0; q < NA; ++q) {
-        const bool ok = q * 16 + m < nv;
-        const int h = hb + (ok ? q * 16 + m : 0);
-        const int a = (h >> 4) & 1;
-        // chunk c (256 bytes) holds steps 2 c and 2 c + 1 (with an odd KS the last holds one);
-        // a 32-row block's chunks are SC / 8 (the padded columns)
+        const uint32_t h = (uint32_t)row[q];
+        const uint32_t at = row[q] >= 0 ? h / 32 * (SC * 32) + (16 * j + h % 16) * 4 : kNoLoad;
 #pragma unroll
-        for (int c = 0; c < (KS + 1) / 2; ++c) {
-          const uint32_t dw = ok ? *(const uint32_t*)(ss + (size_t)(h / 32) * SC * 32 + c * 256 +
-                                                      (16 * j + (h & 15)) * 4)
-                                 : 0x7f7f7f7fu;
-          if constexpr (RAW) {
-            sa[q][2 * c] = dw;
-          } else {
-            sa[q][2 * c] = (dw >> (8 * a)) & 0xffu;
-            if (2 * c + 1 < KS) sa[q][2 * c + 1] = (dw >> (8 * (2 + a))) & 0xffu;
-          }
-        }
+        for (int c = 0; c < (KS + 1) / 2; ++c) sa[q][2 * c] = __builtin_amdgcn_raw_buffer_load_b32(sr, at + c * 256, 0, 0);
       }
     } else {
-      static_assert(KS % 4 == 0, "MXFP4 scales in 16-byte loads");
-      const uint8_t* ss = (const uint8_t*)s;
+      static_assert(WFMT == kFp4 && KS % 4 == 0, "MXFP4 scales in 16-byte loads");
 #pragma unroll
       for (int q = 0; q < NA; ++q) {
-        const bool ok = q * 16 + m < nv;
-        const size_t h = (size_t)hb + (ok ? q * 16 + m : 0);
+        const uint32_t at = row[q] >= 0 ? (uint32_t)row[q] * (KD / 32) : kNoLoad;
 #pragma unroll
         for (int k4 = 0; k4 < KS; k4 += 4) {
-          const u32x4 d = ok ? ld16(ss + h * (KD / 32) + k4 * 4) : u32x4{0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu};
+          const u32x4 d = __builtin_amdgcn_raw_buffer_load_b128(sr, at + k4 * 4, 0, 0);
           const uint32_t dw[4] = {d.x, d.y, d.z, d.w};
 #pragma unroll
-          for (int t = 0; t < 4; ++t) sa[q][k4 + t] = RAW ? dw[t] : (dw[t] >> (8 * j)) & 0xffu;
+          for (int t = 0; t < 4; ++t) sa[q][k4 + t] = dw[t];
         }
       }
     }
@@ -2294,65 +2280,67 @@ struct DownTile {
 #pragma unroll
         for (int w = 0; w < NW; ++w) asm volatile("" : "+v"(a[q][ks][w]));
   }
-  // the scales o requested with load_scales<true> for the unit of first row hb, once they
-  // have landed
-  __device__ __forceinline__ void take_scales(const DownTile& o, int hb, int lane) {
-    const int m = lane & 15, j = lane >> 4;
+  // the scales o requested by load_scales, once they have landed; hi16[q]: whether this lane's A
+  // row of block q lies in the upper half of its 32-row block (the shuffled layout's scales)
+  __device__ __forceinline__ void take_scales(const DownTile& o, const bool (&hi16)[NA], int lane) {
+    const int j = lane >> 4;
+    if constexpr (WFMT == kFp8) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      s0[ks] = o.s0[ks];
-      s1[ks] = o.s1[ks];
-    }
-    if constexpr (WFMT == kFp4 && SH) {
+      for (int ks = 0; ks < KS; ++ks) s0[ks] = o.s0[ks];
+    } else if constexpr (SH) {
 #pragma unroll
       for (int q = 0; q < NA; ++q) {
-        const int a = ((hb + q * 16 + m) >> 4) & 1;  // rows past nv: 0x7f in every byte
+        const uint32_t sh = hi16[q] ? 8u : 0u;
 #pragma unroll
         for (int c = 0; c < (KS + 1) / 2; ++c) {
-          const uint32_t dw = o.sa[q][2 * c];
-          sa[q][2 * c] = (dw >> (8 * a)) & 0xffu;
-          if (2 * c + 1 < KS) sa[q][2 * c + 1] = (dw >> (8 * (2 + a))) & 0xffu;
+          const uint32_t dw = o.sa[q][2 * c] >> sh;
+          sa[q][2 * c] = dw & 0xffu;
+          if (2 * c + 1 < KS) sa[q][2 * c + 1] = (dw >> 16) & 0xffu;
         }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
           if (ks * 128 + 96 >= KR && ks * 128 + 32 * j >= KR) sa[q][ks] = 127u;
       }
-    } else if constexpr (WFMT == kFp4) {
+    } else {
 #pragma unroll
       for (int q = 0; q < NA; ++q)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) sa[q][ks] = (o.sa[q][ks] >> (8 * j)) & 0xffu;
-    } else if constexpr (WFMT == kFp8Mx) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) sa[0][ks] = o.sa[0][ks];
     }
-    split = o.split;
   }
 
-  // w: row 0 of the weight; s: its scales (FP8 [H / 128][KD / 128] fp32, MXFP4 [H][KD / 32])
+  // the shared down's register units: rows [hb, hb + 16) of one weight, nv of them real (hb and nv
+  // multiples of 4). w: row 0 of the weight; s: its scales (fp32 [H / 128][KD / 128], or E8M0
+  // [H / 32][KD / 32])
   __device__ __forceinline__ void load(const uint8_t* w, const void* s, int hb, int nv, int lane) {
-    static_assert(NA == 1 && !SH, "register units are one row-major 16-row block");
+    static_assert(NA == 1 && F8, "register units are one 16-row FP8 block");
     const int m = lane & 15, j = lane >> 4;
     const bool ok = m < nv;
     const size_t h = (size_t)hb + (ok ? m : 0);
-    if constexpr (F8) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const uint8_t* p = w + h * KD + ks * 128 + 16 * j;
+      const bool tail = HALF && ks == KS - 1;  // K 64 .. 127 of the step: past the row
+      if (ok) {
+        a[0][ks][0] = ld16_nt(p);
+        a[0][ks][1] = tail ? u32x4{0u, 0u, 0u, 0u} : ld16_nt(p + 64);
+      } else {
+        a[0][ks][0] = a[0][ks][1] = u32x4{0u, 0u, 0u, 0u};
+      }
+    }
+    if constexpr (WFMT == kFp8) {
+      const float* sp = (const float*)s + (size_t)((hb + min(4 * j, nv - 4)) / 128) * (KD / 128);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) s0[ks] = sp[ks];
+    } else {
+      // lane (m, j) supplies A row hb + m (a unit may straddle two 32-row blocks), its pieces of
+      // step ks in K blocks 4 ks + j / 2 and 4 ks + 2 + j / 2 (the second past the row in a half step)
+      const uint8_t* row = (const uint8_t*)s + (size_t)((hb + min(m, nv - 1)) / 32) * (KD / 32);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        const uint8_t* p = w + h * KD + ks * 128 + 16 * j;
-        const bool tail = HALF && ks == KS - 1;  // K 64 .. 127 of the step: past the row
-        if (ok) {
-          a[0][ks][0] = ld16_nt(p);
-          a[0][ks][1] = tail ? u32x4{0u, 0u, 0u, 0u} : ld16_nt(p + 64);
-        } else {
-          a[0][ks][0] = a[0][ks][1] = u32x4{0u, 0u, 0u, 0u};
-        }
+        const int b0 = 4 * ks + (j >> 1), b1 = b0 + 2;
+        sa[0][ks] = row[b0] | (b1 < KD / 32 ? (uint32_t)row[b1] << 8 : 0u);
       }
-      load_scales(s, hb, nv, lane);
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        a[0][ks][0] = ok ? ld16_nt(w + h * (KD / 2) + ks * 64 + 16 * j) : u32x4{0u, 0u, 0u, 0u};
-      load_scales(s, hb, nv, lane);
     }
   }
 
@@ -2383,9 +2371,9 @@ struct DownTile {
         u32x4 blo = *(const u32x4*)(xr + ks * 128 + 16 * j), bhi = *(const u32x4*)(xr + ks * 128 + 64 + 16 * j);
         const float sx = ((const float*)(xs + row * SST))[ks];
         const f32x4 c = mma_fp8_step(a[0][ks][0], a[0][ks][1], blo, bhi);
-        const float f0 = s0[ks] * sx, f1 = s1[ks] * sx;
+        const float f = s0[ks] * sx;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) acc[0][v] = fmaf(c[v], v < split ? f0 : f1, acc[0][v]);
+        for (int v = 0; v < 4; ++v) acc[0][v] = fmaf(c[v], f, acc[0][v]);
       } else if (scaled) {
         // the scaled MFMA's K layout for the column (see mma_fp4_scaled)
         u32x4 blo = *(const u32x4*)(xr + ks * 128 + 16 * j), bhi = *(const u32x4*)(xr + ks * 128 + 64 + 16 * j);
@@ -3143,7 +3131,8 @@ __device__ __forceinline__ void stage_c(const Params& p, const Union<C>& un, GuS
 // ---------------------------------------------------------------- stage D: shared and routed down + combine
 template <class C>
 struct DownSmem {
-  uint16_t contrib[kRowsMax * C::K * C::TMAX];  // bf16 of a pick's down output x its weight
+  // bf16 of a pick's down output x its weight (8-byte aligned: four rows are stored at once)
+  uint16_t contrib[kRowsMax * C::K * C::TMAX] __attribute__((aligned(16)));
   union {
     struct {
       uint8_t q[C::PB * C::MQS];
@@ -3200,25 +3189,86 @@ __device__ __forceinline__ auto valu_down_loader(const Params& p, const Union<C>
       wr.load(p.w2 + row * (C::I / 2), (const uint8_t*)p.w2_s + row * (C::I / 32), hl < hn, l);
   };
 }
-// request MFMA unit v (slot, 16-row block) of tile rows [h0, h0 + hn), slots from s_lo: its
-// rows into the wave's LDS slot, its scales into nx
+// The MFMA down's units of a pick batch: the tile rows [h0, h0 + hn) of the batch's slots, slot
+// after slot, are one list of ns * hn rows, cut into units of 16 DNA of them. So a unit may hold
+// the last rows of one expert and the first of the next, and no A row is spent on padding a tile
+// to a multiple of 16: a 20-row tile (H 5120) takes 0.625 units of 32 rows an expert instead of
+// one, a 28-row tile (H 7168) 0.875. The picks of a unit's experts are consecutive in the union's
+// order, so they are the unit's columns, 16 a pass; a C value is kept where its row's expert is
+// its column's (the others multiply one expert's rows with another's picks). The down is bound by
+// its waves' converts and MFMAs of whole 16-row blocks, so what it gains is the blocks it no longer
+// runs (us a launch, a tile padded to its own units before): V4.1 TP4 at 8 / 48 rows 75 / 241 ->
+// 70 / 218, TP2 at 8 / 23 rows 116 / 252 -> 108 / 231, TP2 + norm at 48 rows 471 -> 454, FP8 TP4 at
+// 1 / 8 rows 37.0 / 126.6 -> 36.0 / 125.2, MXFP4 TP4 at 8 / 48 rows 81 / 230 -> 80 / 228.
 template <class C>
-__device__ __forceinline__ void mfma_issue(const Params& p, const Union<C>& un, int h0, int hn, int s_lo, int v,
-                                           uint8_t* slot, DownTileOf<C>& nx, int lane) {
+struct DownUnits {
   using DT = DownTileOf<C>;
-  constexpr int UR = 16 * DT::NA;  // rows a unit
-  const int nb = (hn + UR - 1) / UR;
-  const int e = un.slot_e[s_lo + v / nb], rb = v % nb;
-  const int hb = h0 + rb * UR, nv = min(UR, hn - rb * UR);
+  static constexpr int UR = 16 * DT::NA;  // rows a unit
+  int h0, hn, s_lo, ns;
+  // rows a unit takes: UR, or a tile's rows where a unit a slot takes the waves no more rounds (and
+  // more than one): the rounds are then even (TP4 MXFP4 at 2 / 3 / 4 rows 40.2 / 48.7 / 55.5 us with
+  // UR everywhere, 39.8 / 47.8 / 55.2 with this; with one round fewer, fuller units are better: V4.1
+  // TP4 at 1 row 28.3 us against 28.8)
+  int ur;
+  uint32_t inv;  // row / hn = row * inv >> 18 (rows < 4096, hn a multiple of 4 of at most 32)
+  static_assert(C::PB * C::TMAX + 2 * UR <= 4096 && C::TMAX <= 32 && C::TMAX % 4 == 0, "row / hn");
+  __device__ __forceinline__ DownUnits(int h0_, int hn_) : h0(h0_), hn(hn_), s_lo(0), ns(0), ur(UR) {
+    constexpr uint32_t full = ((1u << 18) + C::TMAX - 1) / C::TMAX;  // (a tile's usual rows: no division)
+    inv = hn == C::TMAX ? full : ((1u << 18) + hn - 1) / hn;
+  }
+  __device__ __forceinline__ void slots(int lo, int hi) {
+    s_lo = lo;
+    ns = hi - lo + 1;
+    if constexpr (C::TMAX <= UR)
+      ur = ns > kWaves && (ns + kWaves - 1) / kWaves == (rows() + UR * kWaves - 1) / (UR * kWaves) ? hn : UR;
+  }
+  __device__ __forceinline__ int rows() const { return ns * hn; }
+  __device__ __forceinline__ int units() const {
+    if constexpr (C::TMAX <= UR) return ur == hn ? ns : (rows() + UR - 1) / UR;
+    return (rows() + UR - 1) / UR;
+  }
+  // list row f's slot (from s_lo) and its row of the tile
+  __device__ __forceinline__ int slot(int f) const { return (int)(__umul24((uint32_t)f, inv) >> 18); }
+  __device__ __forceinline__ int tile_row(int f) const { return f - slot(f) * hn; }
+};
+
+// a unit's addresses, read out of the union ahead of its request
+template <class C>
+struct UnitRows {
+  int row[DownTileOf<C>::NA];  // the weight row of this lane's A row of each block (< 0: none)
+  int cblk;                    // FP8: the first block scale of the lane's C rows
+};
+template <class C>
+__device__ __forceinline__ UnitRows<C> unit_rows(const Union<C>& un, const DownUnits<C>& du, int v, int lane) {
+  using DT = DownTileOf<C>;
+  UnitRows<C> u;
+#pragma unroll
+  for (int q = 0; q < DT::NA; ++q) {
+    const int i = q * 16 + (lane & 15), f = v * du.ur + i;
+    const bool ok = i < du.ur && f < du.rows();
+    const int s = du.slot(ok ? f : 0);
+    u.row[q] = ok ? un.slot_e[du.s_lo + s] * C::H + du.h0 + f - s * du.hn : -1;
+  }
+  u.cblk = 0;
+  if constexpr (C::FMT == kFp8) {
+    // the lane's C rows 4 (l / 16) .. + 3 of the unit: one slot, one 128-row scale block (tiles
+    // start and end at multiples of 4)
+    const int f = max(min(v * du.ur + 4 * (lane >> 4), du.rows() - 4), 0), s = du.slot(f);
+    u.cblk = (un.slot_e[du.s_lo + s] * (C::H / 128) + (du.h0 + f - s * du.hn) / 128) * (C::I / 128);
+  }
+  return u;
+}
+// request a unit: its rows into the wave's LDS slot, its scales into nx
+template <class C>
+__device__ __forceinline__ void mfma_issue(const Params& p, const UnitRows<C>& u, uint8_t* slot, DownTileOf<C>& nx,
+                                           int lane) {
+  using DT = DownTileOf<C>;
   static_assert((long long)C::E * C::H * DT::RB < (1ll << 31), "offsets within a 32-bit resource");
-  const auto wr = weight_rsrc(p.w2, (uint32_t)(C::E * C::H * DT::RB));
-  DT::issue(wr, (uint32_t)(e * C::H + hb) * DT::RB, nv, slot, lane);
-  if constexpr (C::FMT == kFp8)
-    nx.load_scales((const float*)p.w2_s + (size_t)e * (C::H / 128) * (C::I / 128), hb, nv, lane);
-  else
-    // (SGLang's layout: the flat [E H][SC] scale matrix's columns are padded to a multiple of 8)
-    nx.template load_scales<true>((const uint8_t*)p.w2_s + (size_t)e * C::H * (C::SHUF ? DT::SC : C::I / 32), hb, nv,
-                                  lane);
+  DT::issue(weight_rsrc(p.w2, (uint32_t)(C::E * C::H * DT::RB)), u.row, slot, lane);
+  // (SGLang's layout: the flat [E H][SC] scale matrix's columns are padded to a multiple of 8)
+  constexpr uint32_t sb = C::FMT == kFp8 ? (uint32_t)C::E * (C::H / 128) * (C::I / 128) * 4
+                                         : (uint32_t)C::E * C::H * (C::SHUF ? DT::SC : C::I / 32);
+  nx.load_scales(weight_rsrc(p.w2_s, sb), u.row, u.cblk, lane);
 }
 
 // picks [pb0, pb0 + pbn) of the union's order, quantized once (stage Q), into the LDS rows of
@@ -3288,7 +3338,7 @@ __device__ __forceinline__ void down_valu(const Params& p, const Union<C>& un, D
   }
 }
 
-// the same on MFMA: units (slot, 16-row block), each against its slot's picks 16 at a time. A
+// the same on MFMA: units of the batch's rows (DownUnits), each against its experts' picks 16 at a time. A
 // wave keeps one unit in flight: once a unit's rows are read out of its LDS slot, the wave's
 // next unit is requested into the slot, and the unit is computed while those rows stream in.
 // Wave w's first unit of a pick batch is unit w (waves 1-7 request it before the hand-offs,
@@ -3301,22 +3351,24 @@ __device__ __forceinline__ void down_mfma(const Params& p, const Union<C>& un, D
   const int npk = p.rows * C::K;
   using DT = DownTileOf<C>;
   constexpr int SST = C::FMT == kFp4 ? C::I / 32 : (C::I / 128) * 4;  // scale bytes of a pick
-  constexpr int UR = 16 * DT::NA;  // rows a unit
-  const int nb = (hn + UR - 1) / UR;
+  DownUnits<C> du(h0, hn);
   uint8_t* slot = sm.wslot[wave];
   int s_lo, s_hi;
   batch_slots(un, 0, min(C::PB, npk), s_lo, s_hi);
   bool ahead = false;  // this wave's first unit of the batch was requested in the batch before
   for (int pb0 = 0; pb0 < npk; pb0 += C::PB) {
     const int pbn = min(C::PB, npk - pb0);
-    const int n_units = (s_hi - s_lo + 1) * nb;
+    du.slots(s_lo, s_hi);
+    const int n_units = du.units();
     // the next batch's slots: a wave's last unit of this batch requests its first unit there,
     // so that the batch change waits for no weight rows
     int nx_lo = 0, nx_hi = -1;
     if (pb0 + C::PB < npk) batch_slots(un, pb0 + C::PB, min(C::PB, npk - pb0 - C::PB), nx_lo, nx_hi);
-    const int nx_units = (nx_hi - nx_lo + 1) * nb;
+    DownUnits<C> dn = du;
+    dn.slots(nx_lo, nx_hi);
+    const int nx_units = dn.units();
     if (!ahead && (pb0 > 0 || first_ready == 0 || (wave == 0 && first_ready < 2)) && wave < n_units)
-      mfma_issue<C>(p, un, h0, hn, s_lo, wave, slot, bt.nxt, lane);
+      mfma_issue<C>(p, unit_rows(un, du, wave, lane), slot, bt.nxt, lane);
     ahead = false;
     const unsigned long long tb0 = tl_now();
     __syncthreads();  // the previous batch is done with the LDS rows (and its claims)
@@ -3334,28 +3386,43 @@ __device__ __forceinline__ void down_mfma(const Params& p, const Union<C>& un, D
     TL_ADD(kTlDQuant, tl_now() - tq0);
     DT cur;
     for (int v = wave; v < n_units;) {
+      // the unit's slots, and the picks (from pb0) of the slot of this lane's C rows of each block
+      const int sa = du.s_lo + du.slot(v * du.ur), sb = du.s_lo + du.slot(min(v * du.ur + du.ur, du.rows()) - 1);
+      const int j0 = max(un.slot_start[sa], pb0), j1 = min(un.slot_start[sb + 1], pb0 + pbn);
+      bool hi16[DT::NA];
+      int c_lo[DT::NA], c_hi[DT::NA], c_hl[DT::NA];
+#pragma unroll
+      for (int q = 0; q < DT::NA; ++q) {
+        const int f = v * du.ur + q * 16;
+        hi16[q] = (((du.h0 + du.tile_row(f + (lane & 15))) >> 4) & 1) != 0;
+        const int fc = f + 4 * (lane >> 4), sc = du.slot(fc);
+        c_hl[q] = fc - sc * hn;
+        const bool ok = q * 16 + 4 * (lane >> 4) < du.ur && sc < du.ns;  // (past the unit's rows: no picks)
+        c_lo[q] = ok ? un.slot_start[du.s_lo + sc] : 0;
+        c_hi[q] = ok ? un.slot_start[du.s_lo + sc + 1] : 0;
+      }
       const unsigned long long tw0 = tl_now();
       wait_vm0();  // the unit's rows are in the slot
       const unsigned long long tf0 = tl_now();
       TL_ADD(kTlDWait, tf0 - tw0);
       TL_ADD(kTlDUnits, 1ull);
-      const int slot_i = s_lo + v / nb, rb = v % nb;
+      // the next unit is claimed once this one's rows are here (a late wave then takes fewer), its
+      // round trip in LDS hidden behind their read-out
+      int nv = 0;
+      if (lane == 0) nv = __hip_atomic_fetch_add(&sm.claim, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       cur.fetch(slot, lane);
-      cur.take_scales(bt.nxt, h0 + rb * UR, lane);
+      cur.take_scales(bt.nxt, hi16, lane);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and read out of it
       const unsigned long long tf1 = tl_now();
       TL_ADD(kTlDFetch, tf1 - tf0);
-      int nv = 0;
-      if (lane == 0) nv = __hip_atomic_fetch_add(&sm.claim, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       nv = __builtin_amdgcn_readfirstlane(nv);
       if (nv < n_units) {
-        mfma_issue<C>(p, un, h0, hn, s_lo, nv, slot, bt.nxt, lane);
+        mfma_issue<C>(p, unit_rows(un, du, nv, lane), slot, bt.nxt, lane);
       } else if (wave < nx_units) {
-        mfma_issue<C>(p, un, h0, hn, nx_lo, wave, slot, bt.nxt, lane);
+        mfma_issue<C>(p, unit_rows(un, dn, wave, lane), slot, bt.nxt, lane);
         ahead = true;
       }
       TL_ADD(kTlDIssue, tl_now() - tf1);
-      const int j0 = max(un.slot_start[slot_i], pb0), j1 = min(un.slot_start[slot_i + 1], pb0 + pbn);
       const int n = lane & 15;
       const unsigned long long tm0 = tl_now();
       for (int jj = j0; jj < j1; jj += kMfmaPicks) {
@@ -3364,13 +3431,13 @@ __device__ __forceinline__ void down_mfma(const Params& p, const Union<C>& un, D
         cur.template mma<C::MQS, SST>(sm.q, sm.s + (GQ ? pick_batch_scales<C>(pb0) : 0u), jj - pb0, np, lane,
                                       C::FMT == kFp4 && p.mx_scaled_down, acc);
         const int pk = n < np ? un.picks[jj + n] : 0;
+        const float w = un.wts[pk];
 #pragma unroll
         for (int q = 0; q < DT::NA; ++q)
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const int hl = rb * UR + q * 16 + 4 * (lane >> 4) + k;
-            if (n < np && hl < hn) sm.contrib[pk * C::TMAX + hl] = f2bf(acc[q][k] * un.wts[pk]);
-          }
+          if (n < np && jj + n >= c_lo[q] && jj + n < c_hi[q])
+            *(u32x2*)(sm.contrib + pk * C::TMAX + c_hl[q]) =
+                u32x2{(uint32_t)f2bf(acc[q][0] * w) | (uint32_t)f2bf(acc[q][1] * w) << 16,
+                      (uint32_t)f2bf(acc[q][2] * w) | (uint32_t)f2bf(acc[q][3] * w) << 16};
       }
       TL_ADD(kTlDMma, tl_now() - tm0);
       if (pb0 == 0 && v == wave) TL(kTlDFirst);
@@ -3394,9 +3461,12 @@ __device__ __forceinline__ void down_first(const Params& p, const Union<C>& un, 
   // these weights (a wave's loads return in order); wave0: wave 0 alone, later
   if ((wave == 0) != wave0) return;
   if constexpr (MF) {
-    constexpr int UR = 16 * DownTileOf<C>::NA;
-    if (wave < (s_hi - s_lo + 1) * ((hn + UR - 1) / UR))
-      mfma_issue<C>(p, un, h0, hn, s_lo, wave, sm.wslot[wave], bt.nxt, threadIdx.x & 63);
+    DownUnits<C> du(h0, hn);
+    du.slots(s_lo, s_hi);
+    if (wave < du.units()) {
+      const int lane = threadIdx.x & 63;
+      mfma_issue<C>(p, unit_rows(un, du, wave, lane), sm.wslot[wave], bt.nxt, lane);
+    }
   } else {
     bt.load(wave, (s_hi - s_lo + 1) * kRowBlocks, valu_down_loader<C>(p, un, h0, hn, s_lo));
   }

@@ -1,0 +1,54 @@
+"""The MFMA down's units against the same rows alone (GPU).
+
+A unit of the routed down holds 16 or 32 rows of the list of a pick batch's experts' tile rows
+(28, 20 or 4 a tile), so it may hold rows of several experts and meet the picks of all of them;
+each value kept is one expert's row against that expert's pick, whose sum no other row, pick or
+unit enters. A step's rows must therefore come out as each row does by itself, bit for bit: one
+row has 6 or 8 experts with one pick each (one unit boundary in each second expert at most), a
+step of many rows every cut of a tile, several pick batches, experts split over two of them and,
+with skewed routing, experts with more picks than an MFMA's 16 columns.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize(
+    "preset,layout,rows,zipf",
+    [
+        ("plumbing_fp8", "row_major", 17, 0.0),  # 4-row tiles: up to five experts a unit
+        ("dsv3_tp4_fp8", "row_major", 2, 0.0),
+        ("dsv3_tp4_fp8", "row_major", 9, 0.0),  # 72 picks: a batch of 64 and one of 8
+        ("dsv3_tp4_fp8", "row_major", 48, 1.2),
+        ("dsv3_tp4_mxfp4", "row_major", 9, 0.0),
+        ("dsv3_tp4_mxfp4", "aiter", 3, 0.0),
+        ("dsv3_tp4_mxfp4", "aiter", 48, 1.2),
+        ("dsv3_tp2_mxfp4_norm", "row_major", 5, 0.0),  # 40 picks: batches of 32
+        ("dsv3_tp2_mxfp4_norm", "aiter", 16, 1.2),
+        ("v41_tp4", "aiter", 2, 0.0),
+        ("v41_tp4", "aiter", 9, 0.0),  # 54 picks: a batch of 51 and one of 3
+        ("v41_tp4", "aiter", 48, 1.2),
+        ("v41_tp2", "aiter", 5, 0.0),  # 30 picks: a batch of 28 and one of 2
+        ("v41_tp2", "aiter", 33, 1.2),
+    ],
+)
+def test_rows_do_not_depend_on_the_step(preset, layout, rows, zipf):
+    from bench import make_layer
+    from sgl_amd_mono.moe.presets import PRESETS
+    from sgl_amd_mono.moe.runner import MoeRunner
+
+    p = PRESETS[preset]
+    g = torch.Generator(device="cuda").manual_seed(97 + rows)
+    w = make_layer(p, g, "cuda", zipf)
+    x = torch.randn(rows, p.hidden, generator=g, device="cuda").to(torch.bfloat16)
+    x[:, 0] = 1.0
+    # (one down kernel at every row count: the scaled MFMA is chosen by the row count)
+    run = MoeRunner(p, layout=layout, mxfp4_scaled_down_rows=49)
+    out = run.moe(w, x)
+    for r in range(rows):
+        alone = run.moe(w, x[r : r + 1])
+        assert torch.equal(out[r], alone[0]), f"row {r} of {rows}"
+    run.raise_on_device_error()
+    assert torch.isfinite(out.float()).all() and out.float().abs().max() > 0
