@@ -2346,8 +2346,10 @@ struct DownTile {
 
   // C tiles (one a 16-row block) against picks [lp, lp + np) of the LDS mid rows (codes xq, row
   // stride QS; scales xs, SST bytes a row: fp32 per 128, or E8M0 per 32)
-  template <int QS, int SST>
-  __device__ __forceinline__ void mma(const uint8_t* xq, const uint8_t* xs, int lp, int np, int lane, bool scaled,
+  // SCALED (MXFP4): on the scaled MFMA. (A parameter of the code, not a branch a K step: the steps are
+  // then one block, whose LDS reads and converts run ahead of the MFMAs of the steps before)
+  template <int QS, int SST, bool SCALED>
+  __device__ __forceinline__ void mma(const uint8_t* xq, const uint8_t* xs, int lp, int np, int lane,
                                       f32x4 (&acc)[NA]) const {
     // (lanes of picks past np read pick lp's row: their output columns are never stored, and
     // an output column depends on its own B column alone)
@@ -2374,7 +2376,7 @@ struct DownTile {
         const float f = s0[ks] * sx;
 #pragma unroll
         for (int v = 0; v < 4; ++v) acc[0][v] = fmaf(c[v], f, acc[0][v]);
-      } else if (scaled) {
+      } else if constexpr (SCALED) {
         // the scaled MFMA's K layout for the column (see mma_fp4_scaled)
         u32x4 blo = *(const u32x4*)(xr + ks * 128 + 16 * j), bhi = *(const u32x4*)(xr + ks * 128 + 64 + 16 * j);
         const uint32_t sx = xs[row * SST + ks * 4 + j];
@@ -2900,7 +2902,7 @@ __device__ __forceinline__ void shared_down_tile(const Params& p, SharedDownSmem
         const int np = min(kMfmaPicks, R - t0);
         f32x4 acc[1];
         dt.opaque();
-        dt.template mma<C::SQS, C::SSC>(sm.q, (const uint8_t*)sm.s, t0, np, lane, false, acc);
+        dt.template mma<C::SQS, C::SSC, false>(sm.q, (const uint8_t*)sm.s, t0, np, lane, acc);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           const int hl = v * 16 + 4 * (lane >> 4) + k;
@@ -3428,8 +3430,9 @@ __device__ __forceinline__ void down_mfma(const Params& p, const Union<C>& un, D
       for (int jj = j0; jj < j1; jj += kMfmaPicks) {
         const int np = min(kMfmaPicks, j1 - jj);
         f32x4 acc[DT::NA];
-        cur.template mma<C::MQS, SST>(sm.q, sm.s + (GQ ? pick_batch_scales<C>(pb0) : 0u), jj - pb0, np, lane,
-                                      C::FMT == kFp4 && p.mx_scaled_down, acc);
+        const uint8_t* xs = sm.s + (GQ ? pick_batch_scales<C>(pb0) : 0u);
+        if (C::FMT == kFp4 && p.mx_scaled_down) cur.template mma<C::MQS, SST, C::FMT == kFp4>(sm.q, xs, jj - pb0, np, lane, acc);
+        else cur.template mma<C::MQS, SST, false>(sm.q, xs, jj - pb0, np, lane, acc);
         const int pk = n < np ? un.picks[jj + n] : 0;
         const float w = un.wts[pk];
 #pragma unroll
