@@ -157,12 +157,9 @@ struct Cfg {
   // (an MX shared expert's width may end in half a 128-K step: V4.1's 2304 / 4 = 576)
   static_assert(I % 128 == 0 && (SFMT == kFp8Mx ? S % 64 == 0 : S % 128 == 0), "widths");
   static_assert(E <= 1024 && (NG == 1 || (E % NG == 0)), "experts");
-  // down-stage mid batch: picks whose quantized rows fit ~32 KB of LDS
-  static constexpr int PB = 32768 / I;
   static constexpr int MQS = I + 16;  // LDS row stride of quantized mid (bank spread)
   static constexpr int SQS = S + 16;
   static constexpr int SSC = SFMT == kFp8Mx ? S / 32 : (S / 128) * 4;  // scale bytes of a shared row
-  static constexpr int MSC = FMT == kFp4 ? I / 32 : I / 128;  // mid scales a pick
   // 16-row blocks of a routed down unit: MXFP4 rows of 512 K are 256 bytes, so a unit of 32 rows
   // keeps 8 KB a wave in flight (as 16 rows do at FP8, or at MXFP4 with 1024 K). At 640 K
   // (V4.1) a tile is H / 256 = 20 rows: one 32-row unit of 10 KB covers it, where 16-row units
@@ -3131,14 +3128,39 @@ __device__ __forceinline__ void stage_c(const Params& p, const Union<C>& un, GuS
 }
 
 // ---------------------------------------------------------------- stage D: shared and routed down + combine
+// The down stage's pick batch: as many picks as their quantized rows (codes and scales) find room for
+// in the CU's LDS beside the union and the rest of the down's. Between two batches every wave waits
+// for the slowest and for the next rows' copy, and an expert whose picks two batches share is read
+// twice, so the fewer batches the better.
+constexpr int kLdsBytes = 160 * 1024;
+template <class C>
+constexpr int pick_scale_bytes() {
+  return C::FMT == kFp4 ? C::I / 32 : (C::I / 128) * 4;
+}
+template <class C>
+constexpr int pick_batch() {
+  constexpr int fixed = kRowsMax * C::K * C::TMAX * 2 + kRowsMax * C::TMAX * 2 + 16 +
+                        kWaves * DownTile<C::FMT, C::I, C::DNA>::SLOT;  // contrib, shv, claim, wslot
+  constexpr int room = kLdsBytes - (int)sizeof(Union<C>) - fixed - 512;  // (512: alignment, small statics)
+  constexpr int n = room / (C::MQS + pick_scale_bytes<C>());
+  return n < kRowsMax * C::K ? n : kRowsMax * C::K;
+}
+// ... and the picks a batch of a step takes: where two batches hold them, two halves (64 picks of at most
+// 54 as 54 and 10, whose few units leave waves idle: TP2 + norm at 8 rows 143 against 140 us)
+template <class C>
+__device__ __forceinline__ int batch_picks(int npk) {
+  constexpr int pb = pick_batch<C>();
+  return npk <= pb ? npk : npk <= 2 * pb ? (npk + 1) / 2 : pb;
+}
 template <class C>
 struct DownSmem {
+  static constexpr int PB = pick_batch<C>();
   // bf16 of a pick's down output x its weight (8-byte aligned: four rows are stored at once)
   uint16_t contrib[kRowsMax * C::K * C::TMAX] __attribute__((aligned(16)));
   union {
     struct {
-      uint8_t q[C::PB * C::MQS];
-      uint8_t s[C::PB * C::MSC * 4];
+      uint8_t q[PB * C::MQS];
+      uint8_t s[PB * pick_scale_bytes<C>() + 16];
     };
     SharedDownSmem<C> sd;  // the shared down's quantized rows, done before the routed ones
   };
@@ -3213,7 +3235,7 @@ struct DownUnits {
   // TP4 at 1 row 28.3 us against 28.8)
   int ur;
   uint32_t inv;  // row / hn = row * inv >> 18 (rows < 4096, hn a multiple of 4 of at most 32)
-  static_assert(C::PB * C::TMAX + 2 * UR <= 4096 && C::TMAX <= 32 && C::TMAX % 4 == 0, "row / hn");
+  static_assert(DownSmem<C>::PB * C::TMAX + 2 * UR <= 4096 && C::TMAX <= 32 && C::TMAX % 4 == 0, "row / hn");
   __device__ __forceinline__ DownUnits(int h0_, int hn_) : h0(h0_), hn(hn_), s_lo(0), ns(0), ur(UR) {
     constexpr uint32_t full = ((1u << 18) + C::TMAX - 1) / C::TMAX;  // (a tile's usual rows: no division)
     inv = hn == C::TMAX ? full : ((1u << 18) + hn - 1) / hn;
@@ -3287,7 +3309,7 @@ template <class C>
 __device__ __forceinline__ void copy_pick_batch(const Params& p, int pb0, int pbn, DownSmem<C>& sm) {
   constexpr uint32_t SST = C::FMT == kFp4 ? C::I / 32 : (C::I / 128) * 4;  // scale bytes of a pick
   static_assert(C::MQS % 16 == 0, "16-byte pieces");
-  static_assert(SST % 16 == 0 || sizeof(sm.s) >= C::PB * SST + 16, "room for the aligned copy");
+  static_assert(sizeof(sm.s) >= DownSmem<C>::PB * SST + 16, "room for the aligned copy");
   ws_to_lds(p, p.off[12] + (uint32_t)pb0 * C::MQS, (uint32_t)pbn * C::MQS, sm.q);
   const uint32_t a = (uint32_t)pb0 * SST - pick_batch_scales<C>(pb0);
   ws_to_lds(p, p.off[13] + a, (uint32_t)(pb0 + pbn) * SST - a, (uint8_t*)sm.s);
@@ -3301,8 +3323,9 @@ __device__ __forceinline__ void down_valu(const Params& p, const Union<C>& un, D
   const int npk = p.rows * C::K;
   using DR = DownRowsOf<C>;
   constexpr int SST = C::FMT == kFp4 ? C::I / 32 : (C::I / 128) * 4;  // scale bytes of a pick
-  for (int pb0 = 0; pb0 < npk; pb0 += C::PB) {
-    const int pbn = min(C::PB, npk - pb0);
+  const int pb = batch_picks<C>(npk);
+  for (int pb0 = 0; pb0 < npk; pb0 += pb) {
+    const int pbn = min(pb, npk - pb0);
     int s_lo, s_hi;
     batch_slots(un, pb0, pbn, s_lo, s_hi);
     const int n_units = (s_hi - s_lo + 1) * kRowBlocks;
@@ -3355,17 +3378,18 @@ __device__ __forceinline__ void down_mfma(const Params& p, const Union<C>& un, D
   constexpr int SST = C::FMT == kFp4 ? C::I / 32 : (C::I / 128) * 4;  // scale bytes of a pick
   DownUnits<C> du(h0, hn);
   uint8_t* slot = sm.wslot[wave];
+  const int pb = batch_picks<C>(npk);
   int s_lo, s_hi;
-  batch_slots(un, 0, min(C::PB, npk), s_lo, s_hi);
+  batch_slots(un, 0, pb, s_lo, s_hi);
   bool ahead = false;  // this wave's first unit of the batch was requested in the batch before
-  for (int pb0 = 0; pb0 < npk; pb0 += C::PB) {
-    const int pbn = min(C::PB, npk - pb0);
+  for (int pb0 = 0; pb0 < npk; pb0 += pb) {
+    const int pbn = min(pb, npk - pb0);
     du.slots(s_lo, s_hi);
     const int n_units = du.units();
     // the next batch's slots: a wave's last unit of this batch requests its first unit there,
     // so that the batch change waits for no weight rows
     int nx_lo = 0, nx_hi = -1;
-    if (pb0 + C::PB < npk) batch_slots(un, pb0 + C::PB, min(C::PB, npk - pb0 - C::PB), nx_lo, nx_hi);
+    if (pb0 + pb < npk) batch_slots(un, pb0 + pb, min(pb, npk - pb0 - pb), nx_lo, nx_hi);
     DownUnits<C> dn = du;
     dn.slots(nx_lo, nx_hi);
     const int nx_units = dn.units();
@@ -3458,7 +3482,7 @@ __device__ __forceinline__ void down_first(const Params& p, const Union<C>& un, 
                                            DownBatchOf<C, MF>& bt, bool wave0 = false) {
   const int npk = p.rows * C::K;
   int s_lo, s_hi;
-  batch_slots(un, 0, min(C::PB, npk), s_lo, s_hi);
+  batch_slots(un, 0, batch_picks<C>(npk), s_lo, s_hi);
   const int wave = (int)(threadIdx.x >> 6);
   // not wave 0, which polls the hand-off next: its flag reads would return only after
   // these weights (a wave's loads return in order); wave0: wave 0 alone, later
