@@ -96,8 +96,25 @@ __global__ __launch_bounds__(kThreads) void k_seam_slice(SeamParams p) {
   const int t0 = blockIdx.y * kTokGroup;
   const int nt = min(kTokGroup, p.T - t0);
 
+  // R, res_out and lin: a thread per (token, column pair); its inputs requested first, so that (a
+  // wave's loads return in order) they are used while the projection's weights still come from HBM
+  const bool rt = tid < nt * (kCols / 2);
+  const int tl0 = rt ? tid / (kCols / 2) : 0, cp = tid % (kCols / 2), col = c0 + 2 * cp, t = t0 + tl0;
+  const uint32_t av = *(const uint32_t*)(p.a + (size_t)t * H + col);
+  uint32_t rv[kHC];
+#pragma unroll
+  for (int h = 0; h < kHC; ++h) rv[h] = *(const uint32_t*)(p.res + ((size_t)t * kHC + h) * H + col);
+  float cm[kHC][kHC], po[kHC], pr[kHC];
+#pragma unroll
+  for (int h = 0; h < kHC; ++h) {
+    po[h] = p.post[t * kHC + h];
+    pr[h] = p.pre[t * kHC + h];
+#pragma unroll
+    for (int oo = 0; oo < kHC; ++oo) cm[h][oo] = p.comb[(t * kHC + h) * kHC + oo];
+  }
+
   // the (projection j, stream o) task of this thread (j = 24: the sum of squares), its 32
-  // weights requested first, into registers
+  // weights into registers
   const int k = tid % 128, half = tid / 128;
   const int j = k / kHC, o = k % kHC;
   f32x4 f[kCols / 4];
@@ -107,21 +124,8 @@ __global__ __launch_bounds__(kThreads) void k_seam_slice(SeamParams p) {
     for (int q = 0; q < kCols / 4; ++q) f[q] = src[q];
   }
 
-  // R, res_out and lin: a thread per (token, column pair)
-  if (tid < nt * (kCols / 2)) {
-    const int tl = tid / (kCols / 2), cp = tid % (kCols / 2), col = c0 + 2 * cp, t = t0 + tl;
-    const uint32_t av = *(const uint32_t*)(p.a + (size_t)t * H + col);
-    uint32_t rv[kHC];
-#pragma unroll
-    for (int h = 0; h < kHC; ++h) rv[h] = *(const uint32_t*)(p.res + ((size_t)t * kHC + h) * H + col);
-    float cm[kHC][kHC], po[kHC], pr[kHC];
-#pragma unroll
-    for (int h = 0; h < kHC; ++h) {
-      po[h] = p.post[t * kHC + h];
-      pr[h] = p.pre[t * kHC + h];
-#pragma unroll
-      for (int oo = 0; oo < kHC; ++oo) cm[h][oo] = p.comb[(t * kHC + h) * kHC + oo];
-    }
+  if (rt) {
+    const int tl = tl0;
     uint32_t ro[kHC] = {0u, 0u, 0u, 0u}, lo = 0u;
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
@@ -239,6 +243,17 @@ __global__ __launch_bounds__(kThreads) void k_seam_gate(SeamParams p) {
     }
   }
 
+  // the gate wave's affine, requested before the partials' sums: after them its two loads (of weights no
+  // cache holds) were a trip to memory in the gate's chain
+  // lane l < 16: comb element (l / 4, l % 4), projection 8 + l; lanes 16 .. 23: pre and post,
+  // projections 0 .. 7; lane 24 and up: the sum of squares
+  const int jj0 = lane < 16 ? 2 * kHC + lane : (lane < kMix ? lane - 16 : kMix);
+  float sc = 0.0f, bs = 0.0f;
+  if (GATE && wave == 0) {
+    sc = p.scale[jj0 < kHC ? 0 : (jj0 < 2 * kHC ? 1 : 2)];
+    bs = p.base[jj0 < kMix ? jj0 : kMix - 1];
+  }
+
   // this token's 25 partials of each slice into LDS, then the group sums: 8 slices in order
   // from the first
   if (GATE) {
@@ -263,9 +278,7 @@ __global__ __launch_bounds__(kThreads) void k_seam_gate(SeamParams p) {
   }
 
   if (GATE && wave == 0) {
-    // lane l < 16: comb element (l / 4, l % 4), projection 8 + l; lanes 16 .. 23: pre and post,
-    // projections 0 .. 7; lane 24 and up: the sum of squares
-    const int jj = lane < 16 ? 2 * kHC + lane : (lane < kMix ? lane - 16 : kMix);
+    const int jj = jj0;
     float mix = red[jj * NG];
 #pragma unroll
     for (int g = 1; g < NG; ++g) mix = mix + red[jj * NG + g];
@@ -273,8 +286,7 @@ __global__ __launch_bounds__(kThreads) void k_seam_gate(SeamParams p) {
     const float dn = __builtin_fmaf(sq, 1.0f / (float)(kHC * H), kMixEps);
     const float rstd = 1.0f / sqrtf(dn);
     const float v = mix * rstd;
-    const int which = jj < kHC ? 0 : (jj < 2 * kHC ? 1 : 2);
-    const float z = __builtin_fmaf(v, p.scale[which], p.base[jj < kMix ? jj : kMix - 1]);
+    const float z = __builtin_fmaf(v, sc, bs);
     if (lane >= 16 && lane < 16 + kHC) p.pre_out[t * kHC + jj] = mkmoe::sigmoid_exact(z) + kHcEps;
     if (lane >= 16 + kHC && lane < kMix) p.post_out[t * kHC + jj - kHC] = mkmoe::sigmoid_exact(z) * kPostMult;
     const bool even_row = ((lane >> 2) & 1) == 0;

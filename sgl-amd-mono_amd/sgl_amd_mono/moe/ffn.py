@@ -131,13 +131,7 @@ class FfnRunner:
         out, res_out, post_out, comb_out, pre_out = outs
         normed = self.normed(m)
         self.seam_runner.ffn_seam(
-            w.seam(), part, residual, post_mix, res_mix, pre_mix, outs=(normed, res_out, post_out, comb_out, pre_out),
-            gate_later=True,
-        )  # fmt: skip
-        try:
-            self.moe_runner.moe(w.moe(), normed, out=out, topk_ids=topk_ids, topk_w=topk_w)
-        except BaseException:
-            self.seam_runner.cancel_gate()
-            raise
-        self.seam_runner.gate()
+            w.seam(), part, residual, post_mix, res_mix, pre_mix, outs=(normed, res_out, post_out, comb_out, pre_out)
+        )
+        self.moe_runner.moe(w.moe(), normed, out=out, topk_ids=topk_ids, topk_w=topk_w)
         return outs
