@@ -390,6 +390,23 @@ __device__ __forceinline__ float tree_sum(float v) {
   return v;
 }
 
+// the halving-tree sums of four values, tree_sum's adds: the first two levels join the values' halves
+// and quarters (permlane32_swap(a, b)[0 / 1]: a's low / high half then b's; permlane16_swap's rows
+// 0 and 2 of a, rows 0 and 2 of b in between), so that the last four levels run once for the four.
+// Lane 0 ends with a's sum, lane 16 with c's, lane 32 with b's, lane 48 with d's
+__device__ __forceinline__ float tree_sum4(float a, float b, float c, float d) {
+  const auto ab = __builtin_amdgcn_permlane32_swap(__float_as_int(a), __float_as_int(b), false, false);
+  const auto cd = __builtin_amdgcn_permlane32_swap(__float_as_int(c), __float_as_int(d), false, false);
+  const float p = __int_as_float((int)ab[0]) + __int_as_float((int)ab[1]);
+  const float q = __int_as_float((int)cd[0]) + __int_as_float((int)cd[1]);
+  const auto pq = __builtin_amdgcn_permlane16_swap(__float_as_int(p), __float_as_int(q), false, false);
+  float v = __int_as_float((int)pq[0]) + __int_as_float((int)pq[1]);
+  v = v + from_lane_above<8>(v);
+  v = v + from_lane_above<4>(v);
+  v = v + from_lane_above<2>(v);
+  return v + from_lane_above<1>(v);
+}
+
 // lane l's value, uniform over the wave
 __device__ __forceinline__ float lane_value(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
@@ -731,25 +748,50 @@ __device__ __forceinline__ void router_unit(const Params& p, RouterSmem<C>& sm, 
   }
   __syncthreads();
   if (e >= C::E) return;
-  for (int r = 0; r < p.rows; ++r) {
+  // The products of bf16 values are exact in fp32, so a fused multiply-add rounds as the product and the
+  // sum do (but where a product leaves fp32's normal range). Rows four at a time share their trees
+  // (tree_sum4) and stores: the sums bound the stage from a few rows on (us a launch, a row at a time
+  // with separate products before: MXFP4 TP4 at 5 / 16 / 48 rows 62.9 / 125.2 / 223.2 -> 61.8 / 123.3 /
+  // 218.5, at 48 rows under Zipf routing 101.5 -> 95.5, V4.1 TP4 at 8 rows 68.7 -> 67.7)
+  float wf[CPP][8];
+#pragma unroll
+  for (int i = 0; i < CPP; ++i) {
+    const uint32_t ww[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      wf[i][2 * q] = bf_lo(ww[q]);
+      wf[i][2 * q + 1] = bf_hi(ww[q]);
+    }
+  }
+  auto row_sum = [&](int r) {
     float acc = 0.0f;
 #pragma unroll
     for (int i = 0; i < CPP; ++i) {
       const u32x4 xv = *(const u32x4*)(sm.x + r * PW + i * 512 + lane * 8);
       const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
-      const uint32_t ww[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        acc = acc + bf_lo(xw[q]) * bf_lo(ww[q]);
-        acc = acc + bf_hi(xw[q]) * bf_hi(ww[q]);
+        acc = __builtin_fmaf(bf_lo(xw[q]), wf[i][2 * q], acc);
+        acc = __builtin_fmaf(bf_hi(xw[q]), wf[i][2 * q + 1], acc);
       }
     }
-    const float s = tree_sum<64>(acc);
-    if (lane == 0) {
-      const uint32_t at = (((uint32_t)r * C::P + part) * C::E + e) * 4;
-      dst32(rs, p.off[5] + at, f2u(s));   // kept for inspection
-      dst32(rs, p.off[10] + at, f2u(s));  // polled, cleared once routed
-    }
+    return acc;
+  };
+  auto put = [&](int r, float s) {
+    const uint32_t at = (((uint32_t)r * C::P + part) * C::E + e) * 4;
+    dst32(rs, p.off[5] + at, f2u(s));   // kept for inspection
+    dst32(rs, p.off[10] + at, f2u(s));  // polled, cleared once routed
+  };
+  int r = 0;
+  // (three last rows too: the fourth's LDS holds whatever it does, its sum is not stored)
+  for (; r + 2 < p.rows; r += 4) {
+    const float s = tree_sum4(row_sum(r), row_sum(r + 1), row_sum(r + 2), row_sum(r + 3));
+    const int g = lane >> 4, rg = r + (g >> 1) + 2 * (g & 1);
+    if ((lane & 15) == 0 && rg < p.rows) put(rg, s);
+  }
+  for (; r < p.rows; ++r) {
+    const float s = tree_sum<64>(row_sum(r));
+    if (lane == 0) put(r, s);
   }
 }
 
@@ -3131,7 +3173,9 @@ __device__ __forceinline__ void stage_c(const Params& p, const Union<C>& un, GuS
 // The down stage's pick batch: as many picks as their quantized rows (codes and scales) find room for
 // in the CU's LDS beside the union and the rest of the down's. Between two batches every wave waits
 // for the slowest and for the next rows' copy, and an expert whose picks two batches share is read
-// twice, so the fewer batches the better.
+// twice, so the fewer batches the better (us a launch, 32 KB of codes a batch before, 28 to 64 picks, and
+// 49 to 108 now: V4.1 TP4 at 48 rows 213.9 -> 208.9, TP2 at 8 rows 105.3 -> 103.9, MXFP4 TP4 at 48 rows
+// under Zipf routing 105.4 -> 100.6, TP2 + norm at 48 rows 440 -> 436).
 constexpr int kLdsBytes = 160 * 1024;
 template <class C>
 constexpr int pick_scale_bytes() {
