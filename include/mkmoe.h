@@ -252,7 +252,8 @@ int mkmoe_clear_errors(const mkmoe_shape* shape, void* ws, size_t ws_bytes, void
  * or fp32 [..][I / 128] scales), 14 / 15 the shared intermediate quantized (above 16 rows,
  * or 24 on the MXFP4 shapes with inter <= 640 and the MX shared expert: codes [rows][S + 16],
  * fp32 scales [rows][S / 128] or E8M0 [rows][S / 32]; below, every workgroup quantizes the
- * shared rows into LDS itself). */
+ * shared rows into LDS itself), 16 the picks as the workgroups poll them (expert int32,
+ * weight fp32: [rows][topk] pairs, every word 0xFFFFFFFF between launches). */
 int mkmoe_workspace_region(const mkmoe_shape* shape, int32_t region, size_t* offset,
                            size_t* bytes);
 

@@ -191,7 +191,7 @@ template <class C>
 __device__ __forceinline__ bool down_on_mfma(int rows, int mfma_down) { return C::SHUF || rows >= mfma_down; }
 
 // ---------------------------------------------------------------- workspace layout
-constexpr int kRegions = 16;
+constexpr int kRegions = 17;
 
 struct Layout {
   size_t off[kRegions];
@@ -224,6 +224,9 @@ MKMOE_HD inline Layout make_layout(int H, int E, int K, int I, int S, int fmt, i
   sz[13] = (size_t)rm * K * (fmt == kFp4 ? I / 32 : (I / 128) * 4);
   sz[14] = (size_t)rm * (S + 16);
   sz[15] = (size_t)rm * (sfmt == kFp8Mx ? S / 32 : (S / 128) * 4);
+  // a pick's expert and weight (8 bytes, written at once) as the workgroups poll them (kPartUnset
+  // between launches)
+  sz[16] = (size_t)rm * K * 8;
   size_t off = kCtlBytes;
   for (int i = 0; i < kRegions; ++i) {
     L.off[i] = off;
@@ -332,6 +335,9 @@ __device__ __forceinline__ u32x4 dld128(__amdgpu_buffer_rsrc_t r, uint32_t off) 
 }
 __device__ __forceinline__ uint32_t dld32(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, kAuxDev);
+}
+__device__ __forceinline__ u32x2 dld64(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, kAuxDev);
 }
 __device__ __forceinline__ uint32_t dld16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, kAuxDev);
@@ -527,10 +533,10 @@ __device__ __forceinline__ void arrive(const Params& p, int which) {
   if (threadIdx.x == 64) dst32(ws_rsrc(p), kCtlFlags + (which * kFlagWgs + blockIdx.x) * 4, 1u);
 }
 
-// wait until the first ``nwg`` workgroups' flags at ``which`` are set (or the deadline
+// wait until the flags at ``which`` of workgroups [from, nwg) are set (or the deadline
 // passed; this workgroup's own flag counts as set, it has arrived): wave 0 reads all of them
 // at once (a lane four); the data behind them is read with sc1 loads afterwards
-__device__ __forceinline__ void await_all(const Params& p, int which, int nwg, int stage) {
+__device__ __forceinline__ void await_all(const Params& p, int which, int nwg, int stage, int from = 0) {
   static_assert(kFlagWgs == 64 * 4, "a lane reads four flags");
   if (threadIdx.x < 64) {
     const auto rs = ws_rsrc(p);
@@ -541,31 +547,11 @@ __device__ __forceinline__ void await_all(const Params& p, int which, int nwg, i
     while (true) {
       const u32x4 f = dld128(rs, off);
       const int i = 4 * lane, own = blockIdx.x;
-      const bool ok = (f.x != 0u || i == own || i >= nwg) && (f.y != 0u || i + 1 == own || i + 1 >= nwg) &&
-                      (f.z != 0u || i + 2 == own || i + 2 >= nwg) && (f.w != 0u || i + 3 == own || i + 3 >= nwg);
+      auto set = [&](uint32_t v, int k) { return v != 0u || k == own || k >= nwg || k < from; };
+      const bool ok = set(f.x, i) && set(f.y, i + 1) && set(f.z, i + 2) && set(f.w, i + 3);
       if (__ballot(!ok) == 0ull && !stall) break;
       if (__builtin_amdgcn_s_memrealtime() - t0 > p.deadline) {
         if (lane == 0) record_error(p, stage, stall);
-        break;
-      }
-    }
-  }
-  __syncthreads();
-}
-
-// wait until workgroup ``wg``'s flag at ``which`` is set (or the deadline passed): wave 0 reads
-// it; the data behind it is read with sc1 loads afterwards
-__device__ __forceinline__ void await_one(const Params& p, int which, int wg, int stage) {
-  if (threadIdx.x < 64) {
-    const auto rs = ws_rsrc(p);
-    const bool stall = stalls(p, stage);
-    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
-    while (true) {
-      // (one address in every lane: a uniform exit)
-      const uint32_t f = __builtin_amdgcn_readfirstlane(dld32(rs, kCtlFlags + (which * kFlagWgs + wg) * 4));
-      if (f != 0u && !stall) break;
-      if (__builtin_amdgcn_s_memrealtime() - t0 > p.deadline) {
-        if (threadIdx.x == 0) record_error(p, stage, stall);
         break;
       }
     }
@@ -861,6 +847,9 @@ __device__ __forceinline__ void reset_parts(const Params& p, int b, int nwg) {
   const int chunks = p.rows * C::P * C::E / 4;
   for (int i = b * kThreads + (int)threadIdx.x; i < chunks; i += nwg * kThreads)
     dst128(rs, p.off[10] + (uint32_t)i * 16, u32x4{kPartUnset, kPartUnset, kPartUnset, kPartUnset});
+  // and the published picks (region 16)
+  for (int i = b * kThreads + (int)threadIdx.x; i < p.rows * C::K; i += nwg * kThreads)
+    dst64(rs, p.off[16] + (uint32_t)i * 8, u32x2{kPartUnset, kPartUnset});
 }
 
 template <class C>
@@ -1202,10 +1191,10 @@ __device__ __forceinline__ void select_row(const Params& p, const RouteSmem<C>& 
 }
 
 // row r's routing by one workgroup (stage B), written to the workspace and the outputs
-template <class C>
+template <class C, bool POLL>
 __device__ __forceinline__ void route_row(const Params& p, RouteSmem<C>& sm, int r) {
   const int lane = threadIdx.x & 63;
-  route_scores<C>(p, sm, r, 1);
+  route_scores<C, POLL>(p, sm, r, 1);
   __syncthreads();
   if (threadIdx.x >= 64) return;
   int id;
@@ -1213,6 +1202,7 @@ __device__ __forceinline__ void route_row(const Params& p, RouteSmem<C>& sm, int
   select_row<C>(p, sm, 0, sm.cv[0], sm.ce[0], sm.ss[0], sm.se[0], lane, id, w);
   if (lane < C::K) {
     const auto rs = ws_rsrc(p);
+    dst64(rs, p.off[16] + (r * C::K + lane) * 8, u32x2{(uint32_t)id, f2u(w)});  // polled
     dst32(rs, p.off[6] + (r * C::K + lane) * 4, (uint32_t)id);
     dst32(rs, p.off[7] + (r * C::K + lane) * 4, f2u(w));
     if (p.ids_out) p.ids_out[r * C::K + lane] = id;
@@ -1245,6 +1235,7 @@ __device__ __forceinline__ void route_all(const Params& p, RouteSmem<C>& sm, int
         wts[r * C::K + lane] = w;
         atomicOr(&rows_of[id][r >> 5], 1u << (r & 31));
         if (publish) {
+          dst64(rs, p.off[16] + (r * C::K + lane) * 8, u32x2{(uint32_t)id, f2u(w)});  // polled
           dst32(rs, p.off[6] + (r * C::K + lane) * 4, (uint32_t)id);
           dst32(rs, p.off[7] + (r * C::K + lane) * 4, f2u(w));
           if (p.ids_out) p.ids_out[r * C::K + lane] = id;
@@ -2436,11 +2427,12 @@ struct DownTile {
 
 // ---------------------------------------------------------------- stage B: routing
 // a workgroup per row (workgroups 0 .. R-1)
-template <class C>
+// (POLL: reading the part sums as they land)
+template <class C, bool POLL = false>
 __device__ __forceinline__ void stage_b(const Params& p, RouteSmem<C>& sm, int b, int nwg) {
   for (int r = b; r < p.rows; r += nwg) {
     __syncthreads();  // the previous row's selection is done with the LDS
-    route_row<C>(p, sm, r);
+    route_row<C, POLL>(p, sm, r);
   }
 }
 
@@ -2475,9 +2467,18 @@ constexpr int kColCost = 2;
 
 // experts picked by any row (ascending id), their picks (pick = row * K + k; a slot's picks
 // in row order, the same in every workgroup) and token groups. The routing comes from
-// un.ids / un.wts when this workgroup routed the step itself (local), else from the workspace.
+// un.ids / un.wts when this workgroup routed the step itself (kRoutedHere), else from the workspace:
+// in the persistent launch each thread polls its pick (kRoutedPolled: expert and weight in one
+// 8-byte word, stored by the workgroup that routed the row), so that no hand-off's flag, its drain
+// before and its read after, stands between the selection and the union (with the part sums
+// polled above 8 rows too: us a launch, with the A and B flags before, MXFP4 TP4 at 48 rows 218.5 ->
+// 214.3, under Zipf routing 96.0 -> 92.4, FP8 TP4 at 33 rows 307.7 -> 303.6, V4.1 TP4 at 48 rows 203.4 ->
+// 201.6, TP2 at 8 rows 103.5 -> 101.6; below, where one workgroup publishes to those of the early
+// shared gate_up: V4.1 TP4 at 8 rows 67.7 -> 66.9, FP8 TP4 at 1 row 36.4 -> 35.7, the DeepSeek-V3 shapes
+// at 3 to 8 rows +0.3 to +1.0); a staged launch reads it (kRoutedBefore)
+enum RoutedBy { kRoutedHere, kRoutedPolled, kRoutedBefore };
 template <class C>
-__device__ __forceinline__ void build_union(const Params& p, Union<C>& un, bool local) {
+__device__ __forceinline__ void build_union(const Params& p, Union<C>& un, RoutedBy by) {
   static_assert(kRowsMax <= 64, "row bitmaps");
   const int tid = threadIdx.x;
   const int npk = p.rows * C::K;
@@ -2489,15 +2490,34 @@ __device__ __forceinline__ void build_union(const Params& p, Union<C>& un, bool 
   static_assert(kRowsMax * C::K <= kThreads, "a pick a thread");
   const int t = tid;
   int my_e = 0;
-  if (local) {
+  if (by == kRoutedHere) {
     if (t < npk) my_e = un.ids[t];
   } else {
     for (int e = tid; e < C::E; e += kThreads) un.rows_of[e][0] = un.rows_of[e][1] = 0u;
     __syncthreads();
+    u32x2 pick = {kPartUnset, kPartUnset};
+    if (by == kRoutedBefore) {
+      if (t < npk) pick = u32x2{dld32(rs, p.off[6] + t * 4), dld32(rs, p.off[7] + t * 4)};
+    } else if ((t & ~63) < npk) {
+      // wave-uniform, as the part sums' poll: until every lane's pick is set, or the deadline
+      // (neither word of a set pick is kPartUnset: a weight that is NaN is the default one)
+      const bool stall = stalls(p, kStageB);
+      const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+      while (true) {
+        const bool wait = t < npk && (pick.x == kPartUnset || pick.y == kPartUnset);
+        if (wait) pick = dld64(rs, p.off[16] + t * 8);
+        if (__ballot(t < npk && (pick.x == kPartUnset || pick.y == kPartUnset)) == 0ull && !stall) break;
+        if (__builtin_amdgcn_s_memrealtime() - t0 > p.deadline) {
+          if ((tid & 63) == 0) record_error(p, kStageB, stall);
+          break;
+        }
+      }
+    }
+    TL(kTlRouted);
     if (t < npk) {
-      my_e = min(max((int)dld32(rs, p.off[6] + t * 4), 0), C::E - 1);
+      my_e = min(max((int)pick.x, 0), C::E - 1);
       un.ids[t] = my_e;
-      un.wts[t] = u2f(dld32(rs, p.off[7] + t * 4));
+      un.wts[t] = u2f(pick.y);
       const int r = t / C::K;
       atomicOr(&un.rows_of[my_e][r >> 5], 1u << (r & 31));
     }
@@ -3641,15 +3661,15 @@ constexpr int shared_mid_rows() {
 
 // the persistent launch past its C arrival: the down stage's first weights depend on the
 // union alone, so they are requested before the wait for the other workgroups' gate_up. GQ
-// (launches of C::QROWS rows or more): stage Q first. PRE: workgroups [0, nsw) ran the shared
-// expert's gate_up in the routing window and set their flags at B, so the first tile's shared
+// (launches of C::QROWS rows or more): stage Q first. PRE: workgroups [w0, w0 + nsw) ran all of the
+// shared expert's gate_up in the routing window and set their flags at B after, so the first tile's shared
 // down runs before the wait (its rows quantized here). MID (with stage Q, up to
 // shared_mid_rows<C>() rows): the first tile's shared down runs inside the Q hand-off, from units
 // in registers, its rows quantized here. Each combination is a code path of its own, so that
 // neither path's registers are allocated around the other's
 template <class C, bool MF, bool GQ, bool PRE = false, bool MID = false>
 __device__ __forceinline__ void wait_then_d(const Params& p, const Union<C>& un, DownSmem<C>& sm, int b, int nwg,
-                                            int nsw = 0) {
+                                            int w0 = 0, int nsw = 0) {
   static_assert(!(MID && PRE), "one place for the shared down");
   static_assert(!MID || (MF && GQ), "the shared down inside the Q hand-off: MFMA down, stage Q");
   DownBatchOf<C, MF> bt;
@@ -3667,7 +3687,7 @@ __device__ __forceinline__ void wait_then_d(const Params& p, const Union<C>& un,
   if (early) down_first<C, MF>(p, un, sm, h0, min(tr, C::H - h0), bt);
   if constexpr (PRE) {
     if (first) {
-      await_all(p, kCtlB, nsw, kStageB);
+      await_all(p, kCtlB, w0 + nsw, kStageB, w0);
       SharedDownBatch<C, MF> bs;
       shared_down_tile<C, MF, false>(p, sm.sd, sm.shv, h0, min(tr, C::H - h0), bs, false);
       // the shared down outlasts most of the gate_up's end spread: wave 0 requests its first
@@ -3737,46 +3757,33 @@ __global__ __launch_bounds__(kThreads) void k_fused(Params p) {
   const int nsw = es.n;
   if (b >= es.w0 && b < es.w0 + es.n) {
     // the shared expert's gate_up while the others route: its weights are requested before
-    // the A hand-off (the x codes) is awaited. Up to 8 rows: then its flag at B (the shared
-    // intermediate stored), and the routing from the workgroup that publishes it; above: its
-    // flag at B first (no row to route), and the routing hand-off after the units
+    // the A hand-off (the x codes) is awaited. Then its flag at B (the shared intermediate is
+    // stored), and the routing as it is published
     int lo, hi;
     even_share(GuDeal<C>::HU * es.k, b - es.w0, es.n, lo, hi);
-    const bool local = p.rows <= local_route_max<C>();
-    if (!local) arrive(p, kCtlB);
     gate_up_shared<C>(p, sm.g, lo, hi, [&] {
       await_all(p, kCtlA, nwg, kStageA);
       TL(kTlAAwaited);
     });
-    if (local) {
-      arrive(p, kCtlB);
-      await_one(p, kCtlB, nwg - 1, kStageB);
-    } else {
-      await_all(p, kCtlB, nwg, kStageB);
-    }
-    TL(kTlRouted);
-    build_union<C>(p, un, false);
+    if (p.rows < C::QROWS) arrive(p, kCtlB);  // (read by the shared down before the C wait alone)
+    build_union<C>(p, un, kRoutedPolled);
     TL(kTlUnion);
   } else if (p.rows <= local_route_max<C>()) {
     // every workgroup routes the step itself, reading the router's part sums as they land:
     // no routing hand-off; the A hand-off (the x codes) is awaited before the gate_up. The
-    // last workgroup publishes the routing (the workspace copies, then its flag at B) for
-    // the workgroups that ran the shared gate_up meanwhile
+    // last workgroup publishes the routing for the workgroups that ran the shared gate_up meanwhile
     route_all<C>(p, sm.r, un.ids, un.wts, un.rows_of, b == nwg - 1);
-    if (nsw > 0 && b == nwg - 1) arrive(p, kCtlB);
     TL(kTlRouted);
-    build_union<C>(p, un, true);
+    build_union<C>(p, un, kRoutedHere);
     TL(kTlUnion);
     await_all(p, kCtlA, nwg, kStageA);
     TL(kTlAAwaited);
   } else {
+    // a workgroup a row routes it, reading the part sums as they land, and publishes its picks
+    stage_b<C, true>(p, sm.r, b, nwg);
     await_all(p, kCtlA, nwg, kStageA);
     TL(kTlAAwaited);
-    stage_b<C>(p, sm.r, b, nwg);
-    arrive(p, kCtlB);
-    await_all(p, kCtlB, nwg, kStageB);
-    TL(kTlRouted);
-    build_union<C>(p, un, false);
+    build_union<C>(p, un, kRoutedPolled);
     TL(kTlUnion);
   }
   stage_c<C>(p, un, sm.g, b, nwg, es);
@@ -3787,11 +3794,11 @@ __global__ __launch_bounds__(kThreads) void k_fused(Params p) {
   if (C::SHUF || down_on_mfma<C>(p.rows, p.mfma_down)) {
     // the shared down before the C wait below stage Q's rows, inside the Q hand-off up to
     // shared_mid_rows<C>() rows, else after the routed down
-    if (nsw > 0 && kPreShared && !gq) {
+    if (nsw > 0 && es.k == GuDeal<C>::shared_units(p.rows) && kPreShared && !gq) {
       // the shared down before the C wait (the shared intermediate was stored in the routing
       // window). (With stage Q, from 8 rows, it cost 1-4 us there against after the routed
       // down or inside the Q hand-off: measured)
-      wait_then_d<C, true, false, true>(p, un, sm.d, b, nwg, nsw);
+      wait_then_d<C, true, false, true>(p, un, sm.d, b, nwg, es.w0, nsw);
     } else if (gq && p.rows <= shared_mid_rows<C>()) {
       wait_then_d<C, true, true, false, true>(p, un, sm.d, b, nwg);
     } else if (gq) {
@@ -3827,20 +3834,20 @@ __global__ __launch_bounds__(kThreads) void k_c(Params p) {
   __shared__ Union<C> un;
   __shared__ GuSmem<C> sm;
   reset_parts<C>(p, blockIdx.x, gridDim.x);  // the routing launch is done with them
-  build_union<C>(p, un, false);
+  build_union<C>(p, un, kRoutedBefore);
   stage_c<C>(p, un, sm, blockIdx.x, gridDim.x);
 }
 template <class C>
 __global__ __launch_bounds__(kThreads) void k_q(Params p) {
   __shared__ Union<C> un;
-  build_union<C>(p, un, false);
+  build_union<C>(p, un, kRoutedBefore);
   if (p.rows >= C::QROWS) stage_q<C>(p, un, blockIdx.x, gridDim.x);
 }
 template <class C>
 __global__ __launch_bounds__(kThreads) void k_d(Params p) {
   __shared__ Union<C> un;
   __shared__ DownSmem<C> sm;
-  build_union<C>(p, un, false);
+  build_union<C>(p, un, kRoutedBefore);
   const bool gq = p.rows >= C::QROWS;
   if (C::SHUF || down_on_mfma<C>(p.rows, p.mfma_down)) {
     DownBatchOf<C, true> bt;
@@ -3940,13 +3947,17 @@ static __device__ __align__(256) uint8_t scratch[kStaticWsBytes];
 
 // before each mkmoe_forward_static launch: the hand-off and error words cleared, the polled
 // router part sums of the call's rows unset (a fill kernel: no memset, so a capture may hold it)
-__global__ void k_static_reset(uint8_t* ws, uint32_t ctl_bytes, uint32_t off10, uint32_t bytes10) {
-  const uint32_t nctl = ctl_bytes / 16, n = nctl + bytes10 / 16;
+// and the published picks (region 16, whole: a multiple of 16 bytes with its padding)
+__global__ void k_static_reset(uint8_t* ws, uint32_t ctl_bytes, uint32_t off10, uint32_t bytes10, uint32_t off16,
+                               uint32_t bytes16) {
+  const uint32_t nctl = ctl_bytes / 16, n10 = nctl + bytes10 / 16, n = n10 + (bytes16 + 15) / 16;
   for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
     if (k < nctl)
       *(u32x4*)(ws + (size_t)k * 16) = u32x4{0u, 0u, 0u, 0u};
-    else
+    else if (k < n10)
       *(u32x4*)(ws + off10 + (size_t)(k - nctl) * 16) = u32x4{kPartUnset, kPartUnset, kPartUnset, kPartUnset};
+    else
+      *(u32x4*)(ws + off16 + (size_t)(k - n10) * 16) = u32x4{kPartUnset, kPartUnset, kPartUnset, kPartUnset};
   }
 }
 
@@ -4150,7 +4161,7 @@ int forward_impl(const mkmoe_shape* s, const mkmoe_weights* w, const void* x, in
   if (static_ws) {
     const uint32_t bytes10 = (uint32_t)rows * s->router_parts * s->experts * 4;
     hipLaunchKernelGGL(k_static_reset, dim3(8), dim3(256), 0, st, (uint8_t*)ws, (uint32_t)kCtlBytes,
-                       (uint32_t)L.off[10], bytes10);
+                       (uint32_t)L.off[10], bytes10, (uint32_t)L.off[16], (uint32_t)L.size[16]);
     if (hipGetLastError() != hipSuccess) return MKMOE_ERR_LAUNCH;
   }
   switch (cfg_id(s)) {
@@ -4201,9 +4212,10 @@ int mkmoe_init_workspace(const mkmoe_shape* shape, void* ws, size_t ws_bytes, vo
   if (!ws) return MKMOE_ERR_NULL;
   if (ws_bytes < layout_of(shape).total) return MKMOE_ERR_WORKSPACE;
   if (hipMemsetAsync(ws, 0, kCtlBytes, (hipStream_t)stream) != hipSuccess) return MKMOE_ERR_HIP;
-  // the polled copy of the router's part sums starts unset (kPartUnset: every byte 0xFF)
+  // the polled copies of the router's part sums and of the picks start unset (kPartUnset: every byte 0xFF)
   const Layout L = layout_of(shape);
-  if (hipMemsetAsync((uint8_t*)ws + L.off[10], 0xFF, L.size[10], (hipStream_t)stream) != hipSuccess)
+  if (hipMemsetAsync((uint8_t*)ws + L.off[10], 0xFF, L.size[10], (hipStream_t)stream) != hipSuccess ||
+      hipMemsetAsync((uint8_t*)ws + L.off[16], 0xFF, L.size[16], (hipStream_t)stream) != hipSuccess)
     return MKMOE_ERR_HIP;
   return MKMOE_OK;
 }

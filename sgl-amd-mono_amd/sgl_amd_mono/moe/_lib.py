@@ -49,6 +49,7 @@ REGIONS = {
     "mid_scales": 13,
     "shared_mid_codes": 14,
     "shared_mid_scales": 15,
+    "picks_polled": 16,
 }
 STAGES = {1: "norm", 2: "router + quantize", 3: "route", 4: "gate_up (routed + shared)", 5: "down (shared + routed) + combine", 6: "quantize the intermediates"}
 

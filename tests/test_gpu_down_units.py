@@ -51,4 +51,6 @@ def test_rows_do_not_depend_on_the_step(preset, layout, rows, zipf):
         alone = run.moe(w, x[r : r + 1])
         assert torch.equal(out[r], alone[0]), f"row {r} of {rows}"
     run.raise_on_device_error()
+    for polled in ("router_parts_polled", "picks_polled"):  # left unset for the next launch
+        assert bool((run.region(polled) == 0xFF).all()), polled
     assert torch.isfinite(out.float()).all() and out.float().abs().max() > 0
