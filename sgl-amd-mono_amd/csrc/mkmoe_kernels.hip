@@ -1980,7 +1980,8 @@ struct GuX {
 
 // this wave's partial C tiles of unit j0 over its K steps: t's weights against x's picks;
 // wsc the FP8 weight's block scales in LDS
-template <class C, int WFMT, bool SH, class StepFn>
+// (ON: on the scaled MFMA (1), converting (0), or as scaled says, a branch a K step (2))
+template <int ON, class C, int WFMT, bool SH, class StepFn>
 __device__ __forceinline__ void gu_mma(const GuTile<C, WFMT, SH>& t, const GuX<C, WFMT>& x, const float* wsc, int W,
                                        int j0, int lane, int wave, bool scaled, f32x4 (&acc)[GuTile<C, WFMT, SH>::NA],
                                        StepFn after_step) {
@@ -2005,7 +2006,7 @@ __device__ __forceinline__ void gu_mma(const GuTile<C, WFMT, SH>& t, const GuX<C
                               e8m0((xe >> (8 * jh)) & 0xffu), e8m0((xe >> (8 * (2 + jh))) & 0xffu), acc[0]);
     } else {
       static_assert(T::NA == 2, "gate and up rows");
-      if (scaled) {
+      if (ON == 1 || (ON == 2 && scaled)) {
         acc[0] = mma_fp4_scaled(t.a[0][i][0], t.sa[0][i], x.lo[i], x.hi[i], x.ex[i], acc[0]);
         acc[1] = mma_fp4_scaled(t.a[1][i][0], t.sa[1][i], x.lo[i], x.hi[i], x.ex[i], acc[1]);
       } else {
@@ -2111,10 +2112,19 @@ __device__ __forceinline__ void gu_mfma(GuSmem<C>& sm, int W, int WR, int lo_h, 
     const unsigned long long tf1 = tl_now();
     TL_ADD(kTlGuFetch, tf1 - tf0);
     f32x4 acc[T::NA];
-    gu_mma<C, WFMT, SH>(t, x, sm.m.wsc, W, j0, lane, wave, scaled, acc, [&](int i) {
+    const auto request = [&](int i) {
       if (more)
         t.issue(wr1, sr1, W, j1, nc1, slot, sslot, lane, wave, i * T::kBlocks / T::SPW, (i + 1) * T::kBlocks / T::SPW);
-    });
+    };
+    // The MFMA chosen once a unit on the narrow MXFP4 shapes (against once a K step, us a launch: TP4 at 1 /
+    // 3 rows 30.7 / 48.2 -> 30.3 / 47.8, V4.1 TP4 at 1 row 27.9 -> 27.6, 8 and 48 rows within noise),
+    // once a K step on the wide ones (once a unit: TP2 + norm at 8 rows +2.2, V4.1 TP2 at 23 rows +1.5)
+    if constexpr (WFMT == kFp4 && C::I <= 640) {
+      if (scaled) gu_mma<1>(t, x, sm.m.wsc, W, j0, lane, wave, scaled, acc, request);
+      else gu_mma<0>(t, x, sm.m.wsc, W, j0, lane, wave, scaled, acc, request);
+    } else {
+      gu_mma<2>(t, x, sm.m.wsc, W, j0, lane, wave, scaled, acc, request);
+    }
 #pragma unroll
     for (int q = 0; q < T::NA; ++q) sm.red[q][wave][lane] = acc[q];
     const unsigned long long tf2 = tl_now();
