@@ -607,7 +607,7 @@ def main() -> int:
                 b = f["alg_MB_per_layer"] * 1e6 + seam_alg_bytes(r)
                 gbps = b / (f["us_per_layer"] * 1e-6) / 1e9
                 res["ffn"] = {
-                    "what": "the FFN: seam (2 launches), MoE block, seam gate, per layer",
+                    "what": "the FFN: seam (2 launches), MoE block, per layer",
                     "us_per_layer": f["us_per_layer"],
                     "us_mean": f["us_mean"],
                     "alg_MB_per_layer": round(b / 1e6, 2),

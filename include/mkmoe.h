@@ -146,8 +146,8 @@ int mkmoe_shape_supported(const mkmoe_shape* shape);
 int mkmoe_workspace_bytes(const mkmoe_shape* shape, size_t* bytes);
 
 /* Zero the workspace's hand-off words (exit count, arrival flags) and error
- * words, and mark the polled router part sums (region 10) unset (enqueued on
- * stream; not for use inside graph capture). Required once before the first
+ * words, and mark the polled router part sums and picks (regions 10 and 16)
+ * unset (enqueued on stream; not for use inside graph capture). Required once before the first
  * forward. */
 int mkmoe_init_workspace(const mkmoe_shape* shape, void* ws, size_t ws_bytes, void* stream);
 

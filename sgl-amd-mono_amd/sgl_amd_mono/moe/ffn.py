@@ -14,9 +14,9 @@ Mirrors the reference's FFN entry point for this path:
 
 The reference runs this as one launch (``gfx950/layer.py:498-598``). Here it is the seam's
 launches (``include/mkmoe_seam.h``) and the MoE's persistent launch (``include/mkmoe.h``) on
-the current stream, in the reference's order: the residual update and the RMSNorm that makes
-the MoE's input first, the MoE on it, and the seam's gate last (the reference runs its gate
-inside the MoE stage, ``layer.py:579-586``). No host synchronisation; outputs and workspaces
+the current stream: the residual update, then the RMSNorm that makes the MoE's input with the
+gate beside it in the same launch, then the MoE (the reference runs its gate inside the MoE
+stage, ``layer.py:579-586``). No host synchronisation; outputs and workspaces
 are allocated on a row count's first call, never inside a graph capture.
 """
 

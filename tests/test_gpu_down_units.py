@@ -20,17 +20,17 @@ pytestmark = pytest.mark.gpu
     [
         ("plumbing_fp8", "row_major", 17, 0.0),  # 4-row tiles: up to five experts a unit
         ("dsv3_tp4_fp8", "row_major", 2, 0.0),
-        ("dsv3_tp4_fp8", "row_major", 9, 0.0),  # 72 picks: a batch of 64 and one of 8
+        ("dsv3_tp4_fp8", "row_major", 16, 0.0),  # 128 picks: two batches of 64
         ("dsv3_tp4_fp8", "row_major", 48, 1.2),
         ("dsv3_tp4_mxfp4", "row_major", 9, 0.0),
         ("dsv3_tp4_mxfp4", "aiter", 3, 0.0),
         ("dsv3_tp4_mxfp4", "aiter", 48, 1.2),
-        ("dsv3_tp2_mxfp4_norm", "row_major", 5, 0.0),  # 40 picks: batches of 32
+        ("dsv3_tp2_mxfp4_norm", "row_major", 8, 0.0),  # 64 picks: two batches of 32
         ("dsv3_tp2_mxfp4_norm", "aiter", 16, 1.2),
         ("v41_tp4", "aiter", 2, 0.0),
-        ("v41_tp4", "aiter", 9, 0.0),  # 54 picks: a batch of 51 and one of 3
+        ("v41_tp4", "aiter", 13, 0.0),  # 78 picks: two batches of 39
         ("v41_tp4", "aiter", 48, 1.2),
-        ("v41_tp2", "aiter", 5, 0.0),  # 30 picks: a batch of 28 and one of 2
+        ("v41_tp2", "aiter", 9, 0.0),  # 54 picks: two batches of 27
         ("v41_tp2", "aiter", 33, 1.2),
     ],
 )
