@@ -3117,7 +3117,7 @@ constexpr bool kPreShared = MKMOE_PRE_SHARED != 0;
 //   - up to local_route_max<C>() rows (every other workgroup routes the step itself): workgroups
 //     [0, n), three quarters of the grid at most, take all k of its units between them (a
 //     unit each where k <= n);
-//   - above (workgroups [0, R) route a row each, then the B hand-off): workgroups [R, R + n)
+//   - above (workgroups [0, R) route a row each, the others poll its picks): workgroups [R, R + n)
 //     take its first k = n units, one each; the others join the routed units' deal.
 // n = 0: none (the shared units are dealt with the routed ones).
 struct EarlyShared {
