@@ -40,6 +40,10 @@ int mkmoe_device_mfma_scaled(const void* a, const void* b, const void* sa, const
 void mkmoe_host_e4m3_encode(const float* x, uint8_t* out, int64_t n);
 void mkmoe_host_sigmoid(const float* x, float* out, int64_t n);
 void mkmoe_host_sqrt_softplus(const float* x, float* out, int64_t n);
+/* the least LDS bytes that the routed down's copies of its pick batches leave of the arrays they go
+ * to, over the batches of a step of rows rows (negative: a copy runs past its array); unit: a
+ * compiled shape (MKMOE_UNIT 0 .. 8; -1 for others) */
+int mkmoe_host_pick_copy_slack(int32_t unit, int32_t rows);
 /* grouped top-k of one row of fp32 scores [E] with fp32 bias */
 void mkmoe_host_topk(const mkmoe_shape* shape, const float* scores, const float* bias,
                      int32_t* ids, float* weights);

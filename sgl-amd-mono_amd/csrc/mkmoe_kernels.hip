@@ -3204,17 +3204,26 @@ __device__ __forceinline__ void stage_c(const Params& p, const Union<C>& un, GuS
 // in the CU's LDS beside the union and the rest of the down's. Between two batches every wave waits
 // for the slowest and for the next rows' copy, and an expert whose picks two batches share is read
 // twice, so the fewer batches the better (us a launch, 32 KB of codes a batch before, 28 to 64 picks, and
-// 49 to 108 now: V4.1 TP4 at 48 rows 213.9 -> 208.9, TP2 at 8 rows 105.3 -> 103.9, MXFP4 TP4 at 48 rows
+// 49 to 107 now: V4.1 TP4 at 48 rows 213.9 -> 208.9, TP2 at 8 rows 105.3 -> 103.9, MXFP4 TP4 at 48 rows
 // under Zipf routing 105.4 -> 100.6, TP2 + norm at 48 rows 440 -> 436).
 constexpr int kLdsBytes = 160 * 1024;
 template <class C>
 constexpr int pick_scale_bytes() {
   return C::FMT == kFp4 ? C::I / 32 : (C::I / 128) * 4;
 }
+// the LDS of n picks' scales: their copy's whole 16-byte pieces (copy_pick_batch), which begin up to 12
+// bytes before the first pick's and end up to 12 after the last's where a pick's are no multiple of 16
+template <class C>
+constexpr int pick_scales_lds(int n) {
+  constexpr int b = pick_scale_bytes<C>();
+  static_assert(b % 4 == 0, "whole words");
+  return (n * b + (b % 16 ? 12 : 0) + 15) / 16 * 16;
+}
 template <class C>
 constexpr int pick_batch() {
   constexpr int fixed = kRowsMax * C::K * C::TMAX * 2 + kRowsMax * C::TMAX * 2 + 16 +
-                        kWaves * DownTile<C::FMT, C::I, C::DNA>::SLOT;  // contrib, shv, claim, wslot
+                        kWaves * DownTile<C::FMT, C::I, C::DNA>::SLOT +  // contrib, shv, claim, wslot
+                        pick_scales_lds<C>(0) + 16;                      // the scales' piece ends
   constexpr int room = kLdsBytes - (int)sizeof(Union<C>) - fixed - 512;  // (512: alignment, small statics)
   constexpr int n = room / (C::MQS + pick_scale_bytes<C>());
   return n < kRowsMax * C::K ? n : kRowsMax * C::K;
@@ -3222,7 +3231,7 @@ constexpr int pick_batch() {
 // ... and the picks a batch of a step takes: where two batches hold them, two halves (64 picks of at most
 // 54 as 54 and 10, whose few units leave waves idle: TP2 + norm at 8 rows 143 against 140 us)
 template <class C>
-__device__ __forceinline__ int batch_picks(int npk) {
+MKMOE_HD inline int batch_picks(int npk) {
   constexpr int pb = pick_batch<C>();
   return npk <= pb ? npk : npk <= 2 * pb ? (npk + 1) / 2 : pb;
 }
@@ -3234,7 +3243,7 @@ struct DownSmem {
   union {
     struct {
       uint8_t q[PB * C::MQS];
-      uint8_t s[PB * pick_scale_bytes<C>() + 16];
+      uint8_t s[pick_scales_lds<C>(PB)];
     };
     SharedDownSmem<C> sd;  // the shared down's quantized rows, done before the routed ones
   };
@@ -3375,18 +3384,25 @@ __device__ __forceinline__ void mfma_issue(const Params& p, const UnitRows<C>& u
 // starts at the 16-byte boundary below the batch's first scale, and the batch's scales begin
 // pick_batch_scales() bytes into sm.s)
 template <class C>
-__device__ __forceinline__ uint32_t pick_batch_scales(int pb0) {
+MKMOE_HD inline uint32_t pick_batch_scales(int pb0) {
   constexpr uint32_t SST = C::FMT == kFp4 ? C::I / 32 : (C::I / 128) * 4;
   return (uint32_t)pb0 * SST % 16;
+}
+// the bytes of sm.s that the copy writes: whole 16-byte pieces
+template <class C>
+MKMOE_HD inline uint32_t pick_batch_scales_end(int pb0, int pbn) {
+  constexpr uint32_t SST = C::FMT == kFp4 ? C::I / 32 : (C::I / 128) * 4;
+  return (pick_batch_scales<C>(pb0) + (uint32_t)pbn * SST + 15) / 16 * 16;
 }
 template <class C>
 __device__ __forceinline__ void copy_pick_batch(const Params& p, int pb0, int pbn, DownSmem<C>& sm) {
   constexpr uint32_t SST = C::FMT == kFp4 ? C::I / 32 : (C::I / 128) * 4;  // scale bytes of a pick
   static_assert(C::MQS % 16 == 0, "16-byte pieces");
-  static_assert(sizeof(sm.s) >= DownSmem<C>::PB * SST + 16, "room for the aligned copy");
+  static_assert(sizeof(sm.s) % 16 == 0 && sizeof(sm.s) >= DownSmem<C>::PB * SST + (SST % 16 ? 12 : 0),
+                "room for the copy's whole pieces");
   ws_to_lds(p, p.off[12] + (uint32_t)pb0 * C::MQS, (uint32_t)pbn * C::MQS, sm.q);
   const uint32_t a = (uint32_t)pb0 * SST - pick_batch_scales<C>(pb0);
-  ws_to_lds(p, p.off[13] + a, (uint32_t)(pb0 + pbn) * SST - a, (uint8_t*)sm.s);
+  ws_to_lds(p, p.off[13] + a, pick_batch_scales_end<C>(pb0, pbn), (uint8_t*)sm.s);
   wait_vm0();
 }
 

@@ -13,17 +13,17 @@ void row(const char* name) {
   using D = DownSmem<C>;
   using G = GuSmem<C>;
   const size_t un = sizeof(Union<C>), st = sizeof(StageSmem<C>);
-  printf("| %s | %d / %d / %d | %zu | %zu | %zu | %zu | %zu | %zu | %zu | %zu | %zu | %zu |\n", name, C::H, C::I,
+  printf("| %s | %d / %d / %d | %zu | %zu | %zu | %zu | %zu | %zu | %zu | %zu | %d | %zu | %zu |\n", name, C::H, C::I,
          C::TMAX, sizeof(RouterSmem<C>), sizeof(RouteSmem<C>), sizeof(G), sizeof(G::m.wslot), sizeof(D),
-         sizeof(D::wslot), sizeof(D::contrib), sizeof(D::shv), un, un + st);
+         sizeof(D::wslot), sizeof(D::contrib), sizeof(D::shv), D::PB, un, un + st);
 }
 
 }  // namespace
 
 int main() {
   printf("| shape | H / I / tile rows | router | routing | gate_up | its weight slots | down | its weight slots "
-         "| pick contributions | shared results | union of experts | launch total |\n");
-  printf("|---|---|---|---|---|---|---|---|---|---|---|---|\n");
+         "| pick contributions | shared results | picks a batch | union of experts | launch total |\n");
+  printf("|---|---|---|---|---|---|---|---|---|---|---|---|---|\n");
   row<mkmoe::CfgPlumbing>("plumbing FP8");
   row<mkmoe::CfgTp4Fp8>("TP4 FP8 (cfg 2)");
   row<mkmoe::CfgTp4Fp4>("TP4 MXFP4 row-major");

@@ -67,6 +67,22 @@ __global__ void k_decode(const uint8_t* codes, float* fp8, float* fp4, int n) {
   }
 }
 
+// the least LDS bytes that a step's copies of its pick batches (copy_pick_batch) leave of their arrays
+template <class C>
+int pick_copy_slack(int rows) {
+  using D = DownSmem<C>;
+  const int npk = rows * C::K, pb = batch_picks<C>(npk);
+  int slack = 1 << 30;
+  for (int pb0 = 0; pb0 < npk; pb0 += pb) {
+    const int pbn = npk - pb0 < pb ? npk - pb0 : pb;
+    const int s = (int)sizeof(D::s) - (int)pick_batch_scales_end<C>(pb0, pbn);
+    const int q = (int)sizeof(D::q) - pbn * C::MQS;
+    slack = s < slack ? s : slack;
+    slack = q < slack ? q : slack;
+  }
+  return slack;
+}
+
 }  // namespace mkmoe
 
 using namespace mkmoe;
@@ -112,6 +128,21 @@ void mkmoe_host_sigmoid(const float* x, float* out, int64_t n) {
 
 void mkmoe_host_sqrt_softplus(const float* x, float* out, int64_t n) {
   for (int64_t i = 0; i < n; ++i) out[i] = sqrt_softplus_exact(x[i]);
+}
+
+int mkmoe_host_pick_copy_slack(int32_t unit, int32_t rows) {
+  switch (unit) {
+    case 0: return pick_copy_slack<CfgPlumbing>(rows);
+    case 1: return pick_copy_slack<CfgTp4Fp8>(rows);
+    case 2: return pick_copy_slack<CfgTp4Fp4>(rows);
+    case 3: return pick_copy_slack<CfgTp2Fp4Norm>(rows);
+    case 4: return pick_copy_slack<CfgTp4Fp4Aiter>(rows);
+    case 5: return pick_copy_slack<CfgTp2Fp4NormAiter>(rows);
+    case 6: return pick_copy_slack<CfgPlumbingSoftplus>(rows);
+    case 7: return pick_copy_slack<CfgV41Tp4>(rows);
+    case 8: return pick_copy_slack<CfgV41Tp2>(rows);
+  }
+  return -1;
 }
 
 void mkmoe_host_topk(const mkmoe_shape* s, const float* scores, const float* bias, int32_t* ids,

@@ -76,6 +76,7 @@ TESTING_EXPORTS = (
     "mkmoe_device_e4m3_sweep",
     "mkmoe_device_mfma_scaled",
     "mkmoe_host_e4m3_encode",
+    "mkmoe_host_pick_copy_slack",
     "mkmoe_host_sigmoid",
     "mkmoe_host_sqrt_softplus",
     "mkmoe_host_topk",
@@ -213,6 +214,7 @@ def testing_lib() -> ctypes.CDLL:
         for name in ("mkmoe_host_e4m3_encode", "mkmoe_host_sigmoid", "mkmoe_host_sqrt_softplus"):
             getattr(T, name).argtypes = [vp, vp, ctypes.c_int64]
             getattr(T, name).restype = None
+        T.mkmoe_host_pick_copy_slack.argtypes = [i32, i32]
         T.mkmoe_host_topk.argtypes = [ctypes.POINTER(Shape), vp, vp, vp, vp]
         T.mkmoe_host_topk.restype = None
         _testing_lib = T

@@ -29,6 +29,7 @@ pytestmark = pytest.mark.gpu
         ("dsv3_tp2_mxfp4_norm", "aiter", 16, 1.2),
         ("v41_tp4", "aiter", 2, 0.0),
         ("v41_tp4", "aiter", 13, 0.0),  # 78 picks: two batches of 39
+        ("v41_tp4", "aiter", 25, 0.0),  # 150 picks: two whole batches of 75, the second's scales off a piece's start
         ("v41_tp4", "aiter", 48, 1.2),
         ("v41_tp2", "aiter", 9, 0.0),  # 54 picks: two batches of 27
         ("v41_tp2", "aiter", 33, 1.2),
