@@ -66,8 +66,8 @@ constexpr int kAuxNt = 2;    // nt: streamed once
 // control words at the start of the workspace: the exit count, the error words; then, from
 // byte kCtlFlags, a flag array per hand-off (a word per workgroup: set on arrival, clear
 // between launches)
-// hand-offs (flag arrays): N normed x, A router and x codes, B routing, C the gate_up, Q the
-// intermediates quantized (the last)
+// hand-offs (flag arrays): N normed x, A router and x codes, B the shared intermediate (where the
+// shared down runs before the C wait), C the gate_up, Q the intermediates quantized (the last)
 constexpr int kCtlNorm = 0, kCtlA = 1, kCtlB = 2, kCtlC = 3, kCtlQ = 4;
 constexpr int kCtlExit = 5;
 constexpr int kCtlErr = 8;  // MKMOE_ERRW_WORDS error words from here
@@ -577,21 +577,24 @@ __device__ __forceinline__ int flags_set_count(const Params& p, int which, int n
   return s_n;
 }
 
-// leave the launch with its flags clear for the next (graph replay safe): every workgroup
-// here has passed the C hand-off (and Q, where the launch has one), so every workgroup has
-// passed the earlier ones and a workgroup clears its own flags of those; the last workgroup
-// out clears the C and Q flags (all have passed those waits) and the exit count
+// leave the launch with its flags clear for the next (graph replay safe). Every workgroup here has
+// passed the C hand-off, so every workgroup has arrived at C, which it does past its N and A waits: a
+// workgroup clears its own flags of those two. The B wait (the shared down before the C wait) comes
+// after a workgroup's arrival at C, as the C and Q waits do, so another workgroup may still be reading
+// B, C and Q here: the last workgroup out clears those (all have passed every wait) and the exit count
 __device__ __forceinline__ void leave(const Params& p) {
   __syncthreads();
   if (threadIdx.x < 64) {
     const auto rs = ws_rsrc(p);
     const int lane = threadIdx.x;
-    if (lane < kCtlC) dst32(rs, kCtlFlags + (lane * kFlagWgs + blockIdx.x) * 4, 0u);
+    static_assert(kCtlNorm == 0 && kCtlA == 1 && kCtlB == 2 && kCtlC == 3 && kCtlQ == 4, "N and A first");
+    if (lane < kCtlB) dst32(rs, kCtlFlags + (lane * kFlagWgs + blockIdx.x) * 4, 0u);
     uint32_t n = 0;
     if (lane == 0)
       n = __hip_atomic_fetch_add(ctl(p) + kCtlExit, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     n = __builtin_amdgcn_readfirstlane(n);
     if (n == gridDim.x - 1) {
+      dst128(rs, kCtlFlags + (kCtlB * kFlagWgs + 4 * lane) * 4, u32x4{0u, 0u, 0u, 0u});
       dst128(rs, kCtlFlags + (kCtlC * kFlagWgs + 4 * lane) * 4, u32x4{0u, 0u, 0u, 0u});
       dst128(rs, kCtlFlags + (kCtlQ * kFlagWgs + 4 * lane) * 4, u32x4{0u, 0u, 0u, 0u});
       if (lane == 0) __hip_atomic_store(ctl(p) + kCtlExit, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -105,3 +105,54 @@ def test_fault_injection_stalls_one_wait(workload, rows, stage, wg):
     torch.cuda.synchronize()
     run.raise_on_device_error()
     assert torch.equal(out2.view(torch.int16), ref.view(torch.int16)), "launch after clear_errors"
+
+
+@pytest.mark.parametrize("preset,layout,rows", [("dsv3_tp4_fp8", "row_major", 4), ("v41_tp2", "aiter", 1)])
+def test_flags_stay_set_while_a_workgroup_still_reads_them(preset, layout, rows):
+    """Below stage Q's rows a workgroup waits at B (the shared intermediate) after its own arrival at
+    C, so the others may pass C, finish and leave while it still reads the B flags: they must stay set
+    until the last workgroup is out. One workgroup's B wait is held for half a second; meanwhile,
+    with the 255 others out, another stream copies the control words to the host."""
+    import time
+
+    from bench import make_layer
+    from sgl_amd_mono.moe.presets import PRESETS
+    from sgl_amd_mono.moe.runner import MoeRunner
+
+    p = PRESETS[preset]
+    g = torch.Generator(device="cuda").manual_seed(31)
+    w = make_layer(p, g, "cuda", 0.0)
+    x = torch.randn(rows, p.hidden, generator=g, device="cuda").to(torch.bfloat16)
+    run = MoeRunner(p, layout=layout, deadline_s=0.5)
+    ref = run.moe(w, x).clone()
+    run.raise_on_device_error()
+    # the control words: the exit count at word 5, from byte 256 the flag arrays N, A, B, C, Q of 256 words
+    words = 64 + 5 * 256
+    host = torch.empty(words, dtype=torch.int32, pin_memory=True)
+    wg = 200  # routes the step itself (the early shared gate_up is on workgroups 0 .. 63 and 0 .. 143)
+    for side in [torch.cuda.Stream() for _ in range(4)]:
+        print(f"\n{preset} R={rows}: workgroup {wg} held at B", flush=True)
+        done = torch.cuda.Event()
+        run.moe(w, x, fault=(3, wg))
+        done.record()
+        time.sleep(0.1)
+        with torch.cuda.stream(side):
+            host.copy_(run.ws.view(torch.int32)[:words], non_blocking=True)
+        side.synchronize()
+        during = not done.query()  # (a stream on the launch's own hardware queue copies after it)
+        torch.cuda.synchronize()
+        e = run.read_errors()
+        run.clear_errors()
+        assert (e[1], e[2], e[4]) == (3, wg, 1), e
+        if during:
+            break
+    else:
+        pytest.fail("every copy waited for the launch")
+    assert int(host[5]) == 255, "the other workgroups are out"
+    n = {"dsv3_tp4_fp8": 64, "v41_tp2": 144}[preset]
+    b = host[64 + 2 * 256 : 64 + 3 * 256]
+    assert bool((b[:n] == 1).all()) and not bool(b[n:].any()), "the B flags"
+    out = run.moe(w, x)
+    run.raise_on_device_error()
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+    assert not bool(run.ws.view(torch.int32)[:words].any()), "the control words are clear between launches"
