@@ -36,6 +36,13 @@ int mkmoe_device_e4m3_sweep(uint32_t first, uint32_t count, uint32_t* bad, uint3
 int mkmoe_device_mfma_scaled(const void* a, const void* b, const void* sa, const void* sb, float* d,
                              int32_t fmt_a, int32_t tiles, void* stream);
 
+/* One workgroup's union of a step of rows rows routed to ids ([rows][topk], any words: as a wait that
+ * gave up may leave them), of a compiled shape (MKMOE_UNIT 0 .. 8): the picks in the union's order
+ * (-1 at a place that it leaves unfilled) and each pick's expert, [rows][topk] words each (device
+ * pointers). */
+int mkmoe_device_union(int32_t unit, int32_t rows, const int32_t* ids, int32_t* picks, int32_t* experts,
+                       void* stream);
+
 /* Host builds of the kernels' exact arithmetic (no device needed): */
 void mkmoe_host_e4m3_encode(const float* x, uint8_t* out, int64_t n);
 void mkmoe_host_sigmoid(const float* x, float* out, int64_t n);

@@ -2528,11 +2528,15 @@ __device__ __forceinline__ void build_union(const Params& p, Union<C>& un, Route
     }
     TL(kTlRouted);
     if (t < npk) {
+      // a row's picks take an expert each, also where a wait that gave up left them unset or half set: the
+      // row bitmaps then count every pick, and the placement below fills every place of un.picks
+      static_assert(C::K <= C::E, "an expert a pick");
+      const int r = t / C::K;
+      const uint32_t bit = 1u << (r & 31);
       my_e = min(max((int)pick.x, 0), C::E - 1);
+      while (atomicOr(&un.rows_of[my_e][r >> 5], bit) & bit) my_e = my_e + 1 < C::E ? my_e + 1 : 0;
       un.ids[t] = my_e;
       un.wts[t] = u2f(pick.y);
-      const int r = t / C::K;
-      atomicOr(&un.rows_of[my_e][r >> 5], 1u << (r & 31));
     }
     __syncthreads();
   }

@@ -83,6 +83,36 @@ int pick_copy_slack(int rows) {
   return slack;
 }
 
+// one workgroup's union of a step whose routing is in the workspace: the picks in the union's order
+// (-1 at a place it leaves unfilled) and each pick's expert
+template <class C>
+__global__ __launch_bounds__(kThreads) void k_union(Params p, int32_t* picks, int32_t* experts) {
+  __shared__ Union<C> un;
+  const int t = threadIdx.x, n = p.rows * C::K;
+  if (t < n) un.picks[t] = -1;
+  build_union<C>(p, un, kRoutedBefore);
+  if (t < n) {
+    picks[t] = un.picks[t];
+    experts[t] = un.ids[t];
+  }
+}
+
+// f(a value of the compiled shape ``unit``'s type)
+template <class F>
+void with_shape(int unit, F f) {
+  switch (unit) {
+    case 0: return f(CfgPlumbing{});
+    case 1: return f(CfgTp4Fp8{});
+    case 2: return f(CfgTp4Fp4{});
+    case 3: return f(CfgTp2Fp4Norm{});
+    case 4: return f(CfgTp4Fp4Aiter{});
+    case 5: return f(CfgTp2Fp4NormAiter{});
+    case 6: return f(CfgPlumbingSoftplus{});
+    case 7: return f(CfgV41Tp4{});
+    case 8: return f(CfgV41Tp2{});
+  }
+}
+
 }  // namespace mkmoe
 
 using namespace mkmoe;
@@ -131,18 +161,26 @@ void mkmoe_host_sqrt_softplus(const float* x, float* out, int64_t n) {
 }
 
 int mkmoe_host_pick_copy_slack(int32_t unit, int32_t rows) {
-  switch (unit) {
-    case 0: return pick_copy_slack<CfgPlumbing>(rows);
-    case 1: return pick_copy_slack<CfgTp4Fp8>(rows);
-    case 2: return pick_copy_slack<CfgTp4Fp4>(rows);
-    case 3: return pick_copy_slack<CfgTp2Fp4Norm>(rows);
-    case 4: return pick_copy_slack<CfgTp4Fp4Aiter>(rows);
-    case 5: return pick_copy_slack<CfgTp2Fp4NormAiter>(rows);
-    case 6: return pick_copy_slack<CfgPlumbingSoftplus>(rows);
-    case 7: return pick_copy_slack<CfgV41Tp4>(rows);
-    case 8: return pick_copy_slack<CfgV41Tp2>(rows);
-  }
-  return -1;
+  int slack = -1;
+  with_shape(unit, [&](auto c) { slack = pick_copy_slack<decltype(c)>(rows); });
+  return slack;
+}
+
+int mkmoe_device_union(int32_t unit, int32_t rows, const int32_t* ids, int32_t* picks, int32_t* experts, void* stream) {
+  if (!ids || !picks || !experts) return MKMOE_ERR_NULL;
+  if (rows < 1 || rows > kRowsMax) return MKMOE_ERR_ROWS;
+  int rc = MKMOE_ERR_SHAPE;
+  with_shape(unit, [&](auto c) {
+    using C = decltype(c);
+    Params p = {};
+    p.rows = rows;
+    p.mfma_gate = 1;
+    p.ws = (uint8_t*)const_cast<int32_t*>(ids);  // ids and, any words, the weights: both are read there
+    p.ws_bytes = (uint32_t)(rows * C::K * 4);
+    hipLaunchKernelGGL(k_union<C>, dim3(1), dim3(kThreads), 0, (hipStream_t)stream, p, picks, experts);
+    rc = hipGetLastError() == hipSuccess ? MKMOE_OK : MKMOE_ERR_LAUNCH;
+  });
+  return rc;
 }
 
 void mkmoe_host_topk(const mkmoe_shape* s, const float* scores, const float* bias, int32_t* ids,

@@ -75,6 +75,7 @@ TESTING_EXPORTS = (
     "mkmoe_device_decode",
     "mkmoe_device_e4m3_sweep",
     "mkmoe_device_mfma_scaled",
+    "mkmoe_device_union",
     "mkmoe_host_e4m3_encode",
     "mkmoe_host_pick_copy_slack",
     "mkmoe_host_sigmoid",
@@ -211,6 +212,7 @@ def testing_lib() -> ctypes.CDLL:
         T.mkmoe_device_decode.argtypes = [vp, vp, vp, i32, vp]
         T.mkmoe_device_e4m3_sweep.argtypes = [ctypes.c_uint32, ctypes.c_uint32, vp, vp, vp]
         T.mkmoe_device_mfma_scaled.argtypes = [vp, vp, vp, vp, vp, i32, i32, vp]
+        T.mkmoe_device_union.argtypes = [i32, i32, vp, vp, vp, vp]
         for name in ("mkmoe_host_e4m3_encode", "mkmoe_host_sigmoid", "mkmoe_host_sqrt_softplus"):
             getattr(T, name).argtypes = [vp, vp, ctypes.c_int64]
             getattr(T, name).restype = None

@@ -5,9 +5,10 @@ routing reads part sums that have not landed (the unset marker, a NaN, so every
 choice is -inf and the row picks experts 0 .. topk-1 with weight 0), the
 hand-offs pass with their data half written, and the launch ends normally. Every
 address a launch derives from hand-off data is clamped (expert ids to [0, E),
-pick slots to the step's picks), so a launch that gave up stays within its
-buffers. The test asserts the error words (code, stage, workgroup, count) and
-that ``clear_errors`` (a full workspace reset) restores a launch bit-identical
+pick slots to the step's picks), and the picks that a workgroup polls take an
+expert each in their row whatever it read, so that its table of them is whole:
+a launch that gave up stays within its buffers. The tests assert the error words
+(code, stage, workgroup, count), the table, and that ``clear_errors`` (a full workspace reset) restores a launch bit-identical
 to a launch on a fresh workspace. The reference's guard test does the same
 from its side (``test/kernels/test_guard_hip.py``, ``common/guard.py:69-89``).
 """
@@ -18,7 +19,41 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("workload,rows", [("cfg2_tp4_fp8", 8), ("cfg2_tp4_fp8", 24), ("cfg3_tp4_mxfp4", 8)])
+@pytest.mark.parametrize("unit,experts,topk", [(0, 16, 4), (1, 256, 8), (7, 384, 6), (8, 384, 6)])
+@pytest.mark.parametrize("rows", [1, 9, 33, 48])
+def test_union_is_whole_whatever_was_read(unit, experts, topk, rows):
+    """Picks as a wait that gave up may leave them (unset, a row half set with the experts that unset
+    ones are clamped to, any words): every place of the union's order holds one pick, and a row's picks
+    have an expert each. Valid picks keep theirs."""
+    from sgl_amd_mono.moe import _lib
+
+    g = torch.Generator().manual_seed(rows)
+    valid = torch.stack([torch.randperm(experts, generator=g)[:topk] for _ in range(rows)]).to(torch.int32)
+    valid[:, 0] = torch.where((valid == 0).any(1), valid[:, 0], 0)  # the expert that unset picks clamp to
+    unset, half = torch.full_like(valid, -1), valid.clone()
+    half[:, topk // 2 :] = -1
+    words = torch.randint(-(2**31), 2**31 - 1, valid.shape, generator=g).to(torch.int32)
+    last = torch.full_like(valid, experts - 1)
+    for name, ids in (("valid", valid), ("unset", unset), ("half", half), ("words", words), ("last", last)):
+        print(f"\nunit {unit} rows {rows}: {name}", flush=True)
+        dev = ids.cuda()
+        picks, got = torch.empty_like(dev), torch.empty_like(dev)
+        rc = _lib.testing_lib().mkmoe_device_union(
+            unit, rows, dev.data_ptr(), picks.data_ptr(), got.data_ptr(), torch.cuda.current_stream().cuda_stream
+        )
+        assert rc == 0
+        got, order = got.cpu(), picks.flatten().cpu()
+        assert bool((got >= 0).all()) and bool((got < experts).all()), name
+        assert all(len(set(r)) == topk for r in got.tolist()), name
+        assert order.tolist() == sorted(range(rows * topk), key=lambda t: (int(got.flatten()[t]), t)), name
+        if name == "valid":
+            assert torch.equal(got, ids)
+
+
+@pytest.mark.parametrize(
+    "workload,rows",
+    [("cfg2_tp4_fp8", 8), ("cfg2_tp4_fp8", 24), ("cfg3_tp4_mxfp4", 8), ("cfg3_tp4_mxfp4", 24), ("cfg5_tp2_mxfp4_norm", 24)],
+)
 def test_deadline_gives_up_then_clear_restores(workload, rows):
     from test_gpu_parity import _case, _runner
 
