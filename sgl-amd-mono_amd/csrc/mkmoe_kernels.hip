@@ -1193,6 +1193,13 @@ __device__ __forceinline__ void select_row(const Params& p, const RouteSmem<C>& 
   my_w = mine_s * f;
 }
 
+// pick t as the workgroups poll it: never the unset word (a weight that is the NaN of all ones, which
+// the caller's scale may be, is published as the NaN below it)
+__device__ __forceinline__ void publish_pick(const Params& p, __amdgpu_buffer_rsrc_t rs, int t, int id, float w) {
+  static_assert(kPartUnset == 0xFFFFFFFFu, "the largest word");
+  dst64(rs, p.off[16] + t * 8, u32x2{(uint32_t)id, min(f2u(w), kPartUnset - 1u)});
+}
+
 // row r's routing by one workgroup (stage B), written to the workspace and the outputs
 template <class C, bool POLL>
 __device__ __forceinline__ void route_row(const Params& p, RouteSmem<C>& sm, int r) {
@@ -1205,7 +1212,7 @@ __device__ __forceinline__ void route_row(const Params& p, RouteSmem<C>& sm, int
   select_row<C>(p, sm, 0, sm.cv[0], sm.ce[0], sm.ss[0], sm.se[0], lane, id, w);
   if (lane < C::K) {
     const auto rs = ws_rsrc(p);
-    dst64(rs, p.off[16] + (r * C::K + lane) * 8, u32x2{(uint32_t)id, f2u(w)});  // polled
+    publish_pick(p, rs, r * C::K + lane, id, w);
     dst32(rs, p.off[6] + (r * C::K + lane) * 4, (uint32_t)id);
     dst32(rs, p.off[7] + (r * C::K + lane) * 4, f2u(w));
     if (p.ids_out) p.ids_out[r * C::K + lane] = id;
@@ -1238,7 +1245,7 @@ __device__ __forceinline__ void route_all(const Params& p, RouteSmem<C>& sm, int
         wts[r * C::K + lane] = w;
         atomicOr(&rows_of[id][r >> 5], 1u << (r & 31));
         if (publish) {
-          dst64(rs, p.off[16] + (r * C::K + lane) * 8, u32x2{(uint32_t)id, f2u(w)});  // polled
+          publish_pick(p, rs, r * C::K + lane, id, w);
           dst32(rs, p.off[6] + (r * C::K + lane) * 4, (uint32_t)id);
           dst32(rs, p.off[7] + (r * C::K + lane) * 4, f2u(w));
           if (p.ids_out) p.ids_out[r * C::K + lane] = id;
@@ -2513,7 +2520,7 @@ __device__ __forceinline__ void build_union(const Params& p, Union<C>& un, Route
       if (t < npk) pick = u32x2{dld32(rs, p.off[6] + t * 4), dld32(rs, p.off[7] + t * 4)};
     } else if ((t & ~63) < npk) {
       // wave-uniform, as the part sums' poll: until every lane's pick is set, or the deadline
-      // (neither word of a set pick is kPartUnset: a weight that is NaN is the default one)
+      // (neither word of a set pick is kPartUnset: publish_pick)
       const bool stall = stalls(p, kStageB);
       const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
       while (true) {

@@ -191,3 +191,28 @@ def test_flags_stay_set_while_a_workgroup_still_reads_them(preset, layout, rows)
     run.raise_on_device_error()
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
     assert not bool(run.ws.view(torch.int32)[:words].any()), "the control words are clear between launches"
+
+
+@pytest.mark.parametrize("rows", [1, 8, 24])
+def test_a_nan_scale_is_no_unset_pick(rows):
+    """Routing weights that are the NaN of all ones (the caller's scale with those bits, carried through
+    the product) are set picks to the workgroups that poll them: the launch ends without a deadline,
+    with the staged launch's output, whose stages read the weights behind each other."""
+    import ctypes
+
+    from test_gpu_parity import _case, _runner
+
+    from sgl_amd_mono.moe import _lib
+
+    c = _case("cfg2_tp4_fp8", 24)
+    x = c.x[:rows].contiguous()
+    run = _runner(c, deadline_s=0.05)
+    at = ctypes.addressof(run.shape) + _lib.Shape.routed_scale.offset
+    ctypes.memmove(at, b"\xff" * 4, 4)
+    wts = torch.zeros(rows, c.preset.topk, device="cuda")
+    out = run.moe(c.w, x, topk_w=wts)
+    run.raise_on_device_error()
+    print(f"\nR={rows}: weights' bits {sorted({hex(v & 0xFFFFFFFF) for v in wts.view(torch.int32).flatten().tolist()})}")
+    staged = run.moe(c.w, x, staged=True)
+    assert torch.equal(out.view(torch.int16), staged.view(torch.int16))
+    assert bool((run.region("picks_polled") == 0xFF).all())
