@@ -1,7 +1,7 @@
 """Parity of the HIP MoE block (through the C ABI) with the CPU oracle, on an MI355X.
 
-Bars: router part sums, activation codes, expert ids and routing weights bit for
-bit at every row count; the bf16 output of every row, against both the oracle's
+Bars: router part sums (but of products below fp32's normal range: a derived bound), activation
+codes, expert ids and routing weights bit for bit at every row count; the bf16 output of every row, against both the oracle's
 exact restatement of the kernel's order and the golden's fp32-matmul form (the
 reference's PyTorch path), within relative L2 1e-2 and max-abs 2e-2 up to the
 bf16 combine's own rounding (gpu_case.within_bar), and cosine 0.9999 against
@@ -10,6 +10,8 @@ fixed-order VALU GEMVs (which the oracle restates) are also bit for bit against 
 and the golden vectors, at small and large row counts. The persistent and the staged
 launches bit for bit alike; repeated and graph-replayed launches bit for bit alike.
 """
+
+import dataclasses
 
 import numpy as np
 import pytest
@@ -37,8 +39,8 @@ CASES = [
     ("cfg2_tp4_fp8", 12),
     ("cfg3_tp4_mxfp4", 12),
     # the last row count every workgroup routes itself (8: the early shared gate_up on
-    # workgroups 0 .. n-1) and the first with the routing hand-off (9: on the workgroups past
-    # the rows); 16 and 17: the shared down inside the Q hand-off and after the routed one
+    # workgroups 0 .. n-1) and the first that a workgroup a row routes and the others poll (9: on
+    # the workgroups past the rows); 16 and 17: the shared down inside the Q hand-off and after the routed one
     ("cfg3_tp4_mxfp4", 9),
     ("cfg3_tp4_mxfp4", 16),
     ("cfg3_tp4_mxfp4", 17),
@@ -46,7 +48,7 @@ CASES = [
     ("tp4_fp8_zipf", 48),
     ("tp2_mxfp4_norm_zipf", 48),
     # V4.1's router scores (sqrt(softplus), one group, check_ffn.py:201-206) on the plumbing
-    # shape: local routing (up to 8 rows) and the routing hand-off (16, 24)
+    # shape: local routing (up to 8 rows) and polled picks (16, 24)
     ("plumbing_fp8_softplus", 1),
     ("plumbing_fp8_softplus", 4),
     ("plumbing_fp8_softplus", 16),
@@ -329,6 +331,39 @@ def test_routing_nan_row(workload, rows):
     assert within_bar(e, len(keep) * c.p["hidden"]), e
 
 
+@pytest.mark.parametrize("workload,rows", [("cfg2_tp4_fp8", 8), ("cfg2_tp4_fp8", 24), ("plumbing_fp8_softplus", 4)])
+def test_router_sums_of_subnormal_products(workload, rows):
+    """The router's fused multiply-adds against the oracle's rounded products where the two differ:
+    products below fp32's normal range. Every value is then under 2^-126, where fp32 is a grid of
+    2^-149 on which sums are exact: the oracle rounds each product to it, a fused add each sum, by
+    half a step at most, so a part sum's PW terms differ by at most PW steps. Logits so near zero
+    score as zero does, and the routing is the oracle's bit for bit."""
+    from oracle import routing as rt
+
+    c = _case(workload, rows)
+    small = lambda t, k: (t.float() * 2.0**k).to(torch.bfloat16)  # noqa: E731 (exact: bf16 has fp32's exponents)
+    x, gate = small(c.x, -68), small(c.w.gate_w, -70)  # products about 2^-145, sums under 2^-130
+    parts = rt.router_part_sums(x.cpu(), gate.cpu(), c.p["router_parts"])
+    scores = rt.score_exact(rt.logits_from_parts(parts), c.p.get("scoring", "sigmoid"))
+    want_ids, want_w = rt.grouped_topk(
+        scores, c.w.bias.cpu().numpy(), c.p["topk"], c.p["n_group"], c.p["topk_group"], c.p["routed_scale"]
+    )
+    run = _runner(c)
+    ids = torch.zeros(rows, c.p["topk"], dtype=torch.int32, device="cuda")
+    wts = torch.zeros(rows, c.p["topk"], dtype=torch.float32, device="cuda")
+    run.moe(dataclasses.replace(c.w, gate_w=gate), x, topk_ids=ids, topk_w=wts)
+    run.raise_on_device_error()
+    e, p = c.p["experts"], c.p["router_parts"]
+    got = run.region("router_parts")[: rows * p * e * 4].view(torch.float32).reshape(rows, p, e).cpu().numpy()
+    want = parts.transpose(0, 2, 1)
+    assert np.abs(want).max() < 2.0**-126 and np.abs(want).max() > 2.0**-149 * 64  # subnormal, and not all zero
+    diff = np.abs(got.astype(np.float64) - want).max() / 2.0**-149
+    print(f"\n{workload} R={rows}: part sums differ by up to {diff:.0f} steps of 2^-149", flush=True)
+    assert diff <= c.p["hidden"] // p
+    assert np.array_equal(ids.cpu().numpy(), want_ids), "expert ids"
+    assert np.array_equal(wts.cpu().numpy().view(np.uint32), want_w.view(np.uint32)), "routing weights"
+
+
 def gen_dense(c):
     from oracle import gen
 
@@ -386,9 +421,9 @@ def test_staged_equals_fused_and_repeats(workload, rows):
 
 
 def test_row_counts_in_turn_on_one_workspace():
-    """Launches of changing row counts (local routing and the routing hand-off in turn) on one
-    runner: each launch must find the hand-off flags and the polled part sums as the previous
-    one left them, and be checked against its own oracle case."""
+    """Launches of changing row counts (local routing and polled picks in turn) on one
+    runner: each launch must find the hand-off flags, the polled part sums and the polled picks as
+    the previous one left them, and be checked against its own oracle case."""
     run = None
     for rows in (4, 20, 1, 16, 3):
         c = _case("cfg1_plumbing_fp8", rows)
@@ -444,7 +479,7 @@ def test_device_e4m3_convert_equals_encoder_on_every_float():
 
 
 def test_graph_replay_bitwise_routing_handoff():
-    """Rows 24 and 48 (the routing hand-off, stage Q) in one graph, replayed with eager work between."""
+    """Rows 24 and 48 (polled picks, stage Q) in one graph, replayed with eager work between."""
     c = _case("cfg2_tp4_fp8", 48)
     run = _runner(c)
     rows = (24, 48)

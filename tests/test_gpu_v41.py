@@ -166,7 +166,7 @@ def test_v41_staged_equals_fused_and_repeats(workload, rows):
 
 @pytest.mark.parametrize("workload", [WORKLOAD, TP2])
 def test_v41_graph_replay_bitwise(workload):
-    """Row counts on both sides of the routing hand-off and of stage Q in one graph, replayed
+    """Row counts on both sides of the local routing's limit and of stage Q in one graph, replayed
     with eager work between the replays."""
     c = _case(48, workload)
     run = _runner(c)
@@ -199,8 +199,8 @@ def test_v41_graph_replay_bitwise(workload):
 
 @pytest.mark.parametrize("rows", [1, 8, 48])
 def test_v41_ffn_chain(rows):
-    """The FFN entry point (``FfnRunner.ffn``: the seam, the MoE block on the seam's normed
-    rows, then the seam's gate) against its parts: every seam output bit for bit the seam's
+    """The FFN entry point (``FfnRunner.ffn``: the seam with its gate, then the MoE block on the
+    seam's normed rows) against its parts: every seam output bit for bit the seam's
     own launch's, the partial bit for bit the MoE launch's on those normed rows, and the
     routing of the normed rows the oracle's; then a captured graph of the call, replayed."""
     from oracle import gen
