@@ -192,8 +192,8 @@ class RowsBench:
 
 
 class FfnRowsBench(RowsBench):
-    """DeepSeek-V4.1's FFN at one row count (``FfnRunner.ffn``: the seam, the MoE block on its
-    normed rows, the seam's gate), over the MoE layers' weights with a seam weight set each."""
+    """DeepSeek-V4.1's FFN at one row count (``FfnRunner.ffn``: the seam with its gate, the MoE block on its
+    normed rows), over the MoE layers' weights with a seam weight set each."""
 
     def __init__(self, ffn, layers, seam_ws, preset, rows, device, seed):
         import torch
@@ -562,7 +562,7 @@ def main() -> int:
         if preset.routed_fmt == "mxfp4" and not preset.aiter_only:
             kw["layout"] = args.layout
         runner = MoeRunner(preset, device, max_rows=max(48, max(rows_list)), **kw)
-        # V4.1: its whole FFN too (the seam, the MoE block, the seam's gate) on the same weights
+        # V4.1: its whole FFN too (the seam with its gate, the MoE block) on the same weights
         ffn = None
         if preset.hidden == SEAM_H and preset.aiter_only and not (args.staged or args.timeline or args.no_ffn):
             from sgl_amd_mono.moe.ffn import FfnRunner
@@ -613,7 +613,7 @@ def main() -> int:
                     "alg_MB_per_layer": round(b / 1e6, 2),
                     "GBps": round(gbps, 1),
                     "pct_hbm_peak": round(100 * gbps / HBM_PEAK_GBPS, 2),
-                    "launches_timed": 4 * f["launches_timed"],
+                    "launches_timed": 3 * f["launches_timed"],
                 }
                 del fb
             wres[str(r)] = res
