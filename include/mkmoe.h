@@ -70,7 +70,8 @@ extern "C" {
                               * or, with a fault injected, the stalled wait's: the waits it
                               * holds up downstream may reach their deadlines before it) */
 #define MKMOE_ERRW_BLOCK 2   /* the workgroup that saw it */
-#define MKMOE_ERRW_COUNT 3   /* how many waits ran past their deadline */
+#define MKMOE_ERRW_COUNT 3   /* how many waits ran past their deadline (a wait on flags counts once a
+                              * workgroup, a poll of part sums or picks once a wave) */
 #define MKMOE_ERRW_FAULT 4   /* 1: a wait stalled by mkmoe_options.fault_stage ran to its deadline */
 #define MKMOE_ERRW_WORDS 8
 #define MKMOE_DEVERR_DEADLINE 1
@@ -215,7 +216,7 @@ int mkmoe_forward_staged(const mkmoe_shape* shape, const mkmoe_weights* w, const
  * compiled shape at 48 rows; a larger layout returns MKMOE_ERR_WORKSPACE) lives
  * in each GPU the library runs on until the process ends. Each call enqueues a
  * small fill kernel that clears the array's hand-off and error words and marks
- * the call's polled router part sums unset, then the forward kernel: two
+ * the call's polled router part sums and picks unset, then the forward kernel: two
  * launches, both safe to capture. Every call on one GPU shares that GPU's
  * array, so calls that may overlap on one GPU (other streams, other threads)
  * race and must not be issued. Its device error words are not readable
@@ -228,12 +229,12 @@ int mkmoe_forward_static(const mkmoe_shape* shape, const mkmoe_weights* w, const
 /* Copy the MKMOE_ERRW_WORDS error words to host memory (synchronises stream).
  * After a device error (MKMOE_ERRW_CODE non-zero) the launch that recorded it
  * gave up waiting, so its output is not valid and its hand-off state (arrival
- * flags, the polled router part sums) may be left half set: call
+ * flags, the polled router part sums and picks) may be left half set: call
  * mkmoe_clear_errors before the next forward on that workspace. */
 int mkmoe_read_errors(const void* ws, int32_t* words, int32_t n, void* stream);
 
-/* Reset a workspace after a device error: the error words, the hand-off words
- * and the polled router part sums, as mkmoe_init_workspace does (enqueued on
+/* Reset a workspace after a device error: the error words, the hand-off words,
+ * the polled router part sums and picks, as mkmoe_init_workspace does (enqueued on
  * stream; not for use inside graph capture). */
 int mkmoe_clear_errors(const mkmoe_shape* shape, void* ws, size_t ws_bytes, void* stream);
 

@@ -161,9 +161,9 @@ struct Cfg {
   static constexpr int SQS = S + 16;
   static constexpr int SSC = SFMT == kFp8Mx ? S / 32 : (S / 128) * 4;  // scale bytes of a shared row
   // 16-row blocks of a routed down unit: MXFP4 rows of 512 K are 256 bytes, so a unit of 32 rows
-  // keeps 8 KB a wave in flight (as 16 rows do at FP8, or at MXFP4 with 1024 K). At 640 K
-  // (V4.1) a tile is H / 256 = 20 rows: one 32-row unit of 10 KB covers it, where 16-row units
-  // took two, the second with 4 rows at a whole unit's latency
+  // keeps 8 KB a wave in flight (as 16 rows do at FP8, or at MXFP4 with 1024 K), at 640 K (V4.1)
+  // 10 KB. Units are cut across the experts' tile rows (DownUnits), so a tile's rows (20 or 28) need
+  // not be a multiple of a unit's
   static constexpr int DNA = FMT == kFp4 && I <= 640 ? 2 : 1;
   static constexpr int TMAX = tile_max(H);  // output rows of a down tile, at most
 };
@@ -711,8 +711,8 @@ struct RouterSmem {
 
 // router part sums of one workgroup unit: K part ``part`` of experts eb * 8 .. eb * 8 + 7
 // (one a wave) for every row, in the fixed order: lane l sums its 8 columns of each
-// 512-column chunk of the part in order (products rounded, then added), then the
-// wave's halving tree
+// 512-column chunk of the part in order by fused multiply-adds (as products rounded, then
+// added, but where a product leaves fp32's normal range), then the wave's halving tree
 template <class C>
 __device__ __forceinline__ void router_unit(const Params& p, RouterSmem<C>& sm, int part, int eb, int lane, int wave,
                                             const float* rstd) {
@@ -891,9 +891,9 @@ __device__ __forceinline__ void stage_a(const Params& p, RouterSmem<C>& sm, int 
 // ---------------------------------------------------------------- stage B: routing
 // Scores and choices of kRouteRows rows at a time, in LDS
 constexpr int kRouteRows = 16;
-// rows up to which every workgroup routes the whole step itself (no routing hand-off). Above,
-// a workgroup a row and the hand-off cost less than every workgroup's scores of all the rows:
-// 8 against 16 at 12 and 16 rows, cfg 2 -2.8 / -3.4 us, cfg 3 -3.6 / -5.6, V4.1 TP4 -6.1 /
+// rows up to which every workgroup routes the whole step itself. Above, a workgroup a row, whose
+// picks the others poll, costs less than every workgroup's scores of all the rows (measured where the
+// others still waited for flags): 8 against 16 at 12 and 16 rows, cfg 2 -2.8 / -3.4 us, cfg 3 -3.6 / -5.6, V4.1 TP4 -6.1 /
 // -5.4 (its 384 sqrt(softplus) scores a row); lower, mixed, but V4.1 at TP2 gains with 4
 // (-0.6 / -1.6 / -1.8 us at 5 / 6 / 8 rows: measured)
 constexpr int kLocalRouteMax = 8;

@@ -292,7 +292,7 @@ class MoeRunner:
 
     def clear_errors(self) -> None:
         """Reset the workspace after a device error: the error words, and the hand-off state
-        (flags, polled router part sums) that a launch cut short by a deadline may leave."""
+        (flags, polled router part sums and picks) that a launch cut short by a deadline may leave."""
         no_capture("a workspace reset")
         _lib.check(
             self.lib.mkmoe_clear_errors(ctypes.byref(self.shape), self.ws.data_ptr(), self.ws.numel(), self._stream()),
